@@ -220,8 +220,8 @@ int kata_gemv_q8_0_batch(int count, const uint8_t* const* W, float* const* y, co
 }
 
 // ------------------------------------------------------------------ prefill
-int kata_gemm_ptq1_f16(const uint16_t* A, int lda, const uint8_t* W, void* C, int c_dtype, int ldc, int M, int K,
-                       int N, void* stream) {
+static int check_gemm_f16_args(const uint16_t* A, int lda, const uint8_t* W, const void* C, int c_dtype, int ldc, int M,
+                               int K, int N) {
     if (!A || !W || !C) return fail(KATA_EINVAL, "null pointer argument");
     if (M <= 0 || N <= 0) return fail(KATA_EINVAL, "M=%d N=%d must be positive", M, N);
     if (K <= 0 || K % 128 != 0) return fail(KATA_EINVAL, "K=%d must be a positive multiple of 128", K);
@@ -230,6 +230,12 @@ int kata_gemm_ptq1_f16(const uint16_t* A, int lda, const uint8_t* W, void* C, in
     if (c_dtype != KATA_F32 && c_dtype != KATA_F16) return fail(KATA_EINVAL, "c_dtype=%d", c_dtype);
     if (!aligned(A, 16)) return fail(KATA_EINVAL, "A must be 16-byte aligned");
     if (!aligned(W, 2)) return fail(KATA_EINVAL, "W must be 2-byte aligned");
+    return KATA_OK;
+}
+
+int kata_gemm_ptq1_f16(const uint16_t* A, int lda, const uint8_t* W, void* C, int c_dtype, int ldc, int M, int K,
+                       int N, void* stream) {
+    if (int rc = check_gemm_f16_args(A, lda, W, C, c_dtype, ldc, M, K, N)) return rc;
     return check_launch(kata::launch_gemm_f16(A, lda, W, C, c_dtype, ldc, M, K, N, (hipStream_t)stream),
                         "gemm ptq1 f16");
 }
@@ -574,6 +580,27 @@ int kata_dispatch_prefill(kata_dispatch* d, uint64_t wOff, const uint16_t* A, fl
 }
 
 
+namespace {
+// The fp32 outputs C[i] [M][N[i]] of the named matrices that are not selected for int8, all
+// reading the fp16 rows A [M][K], as one launch.
+int prefill_f16_batch(kata_dispatch* d, int count, const uint64_t* offs, const char* const* names, float* const* outs,
+                      const int* N, const uint16_t* A, int M, int K, void* stream) {
+    const uint8_t* W[4];
+    void* C[4];
+    int Nf[4], n = 0;
+    for (int i = 0; i < count; i++) {
+        if (kata_dispatch_i8(d, names[i])) continue;
+        if (int rc = check_gemm_f16_args(A, K, d->wbase + offs[i], outs[i], KATA_F32, N[i], M, K, N[i])) return rc;
+        W[n] = d->wbase + offs[i];
+        C[n] = outs[i];
+        Nf[n++] = N[i];
+    }
+    if (!n) return KATA_OK;
+    return check_launch(kata::launch_gemm_f16_multi(A, K, n, W, C, KATA_F32, Nf, M, K, Nf, (hipStream_t)stream),
+                        "gemm ptq1 f16 batch");
+}
+}  // namespace
+
 // ------------------------------------------------------------------ layer-level: the FFN sublayer
 // Engine::step's FFN (src/engine.cpp:176-182): h = H(rmsnorm(x + y) * gs_in) (the residual
 // x + y is kept in xnew), g = W_gate h, u = W_up h (one batched launch), t = H(silu(g) u *
@@ -617,8 +644,15 @@ int kata_dispatch_ffn_prefill(kata_dispatch* d, uint64_t offGate, uint64_t offUp
     float* SX = (float*)(((uintptr_t)(A8 + (size_t)M * kmax) + 15) & ~(uintptr_t)15);
     int rc = kata_add_rms_fwht(x, y, gs_in, h, KATA_F16, KATA_X_ROWS, xnew, nullptr, nullptr, 0, H, M, stream);
     if (rc) return rc;
-    if ((rc = kata_dispatch_prefill(d, offGate, h, g, M, H, F, "gate", A8, SX, M, stream))) return rc;
-    if ((rc = kata_dispatch_prefill(d, offUp, h, u, M, H, F, "up", A8, SX, M, stream))) return rc;
+    const uint64_t offs[2] = {offGate, offUp};
+    const char* const names[2] = {"gate", "up"};
+    float* const gu[2] = {g, u};
+    const int Ng[2] = {F, F};
+    if ((rc = prefill_f16_batch(d, 2, offs, names, gu, Ng, h, M, H, stream))) return rc;
+    for (int i = 0; i < 2; i++)
+        if (kata_dispatch_i8(d, names[i]) &&
+            (rc = kata_dispatch_prefill(d, offs[i], h, gu[i], M, H, F, names[i], A8, SX, M, stream)))
+            return rc;
     if ((rc = kata_rms_fwht(g, u, gs_down, t, KATA_F16, KATA_X_ROWS, F, M, 1, stream))) return rc;
     return kata_dispatch_prefill(d, offDown, t, out, M, F, H, "down", A8, SX, M, stream);
 }
@@ -730,10 +764,12 @@ int kata_dispatch_in(kata_dispatch* d, int form, int count, const uint64_t* offs
         if (form == KATA_FORM_DECODE) return kata_gemv_ptq1_batch(count, Wm, outs, N, w.act, KATA_XQ, KATA_X_ROWS, H, 1, stream);
         return kata_gemv_ptq1_wide_batch(count, Wm, outs, N, w.act, KATA_XQ, H, M, stream);
     }
-    bool quantised = false;                          // prefill: quantise h once for its int8 matrices
+    if ((rc = prefill_f16_batch(d, count, offs, names, outs, N, (const uint16_t*)w.act, M, H, stream))) return rc;
+    bool quantised = false;                          // quantise h once for its int8 matrices
     for (int i = 0; i < count; i++) {
+        if (!kata_dispatch_i8(d, names[i])) continue;
         if ((rc = half_matmul(d, form, offs[i], names[i], w, outs[i], H, N[i], M, quantised, st))) return rc;
-        quantised = quantised || (form == KATA_FORM_PREFILL && kata_dispatch_i8(d, names[i]));
+        quantised = true;
     }
     return KATA_OK;
 }

@@ -5,196 +5,219 @@
 // half(trit*d) is exact, so every product term equals the reference's; only the fp32
 // summation order differs (tolerance-based parity).
 //
-// Design (MI355X-first; the reference expands every matrix to a 178 MB fp16 stage first):
-//  * Work is cut into tiles of 256 rows of A / C by 128 columns (8 units of 16).  Tiles are
-//    taken whole by one workgroup each for as many full rounds of the CU count as there
-//    are; the tiles left over are split along K into pieces, one workgroup each, so the
-//    last round fills the chip too.  A piece writes its fp32 partial tile to a workspace
-//    and a second kernel adds the pieces of each tile in piece order (deterministic).
-//    256-row tiles halve the weight decoding per flop against 128-row ones.  K advances in
-//    stages of 64 (half a PTQ1_0 block).
-//  * 8 waves, two per SIMD.  Waves 0..3 are consumers: wave w owns rows 64w..64w+63 and all
-//    128 columns, 2 x 4 tiles of v_mfma_f32_32x32x16_f16, with the A and B fragments of a
-//    16-k step loaded from LDS before the MFMAs of the step before it.  Waves 4..7 are producers:
-//    they copy A tiles into LDS by DMA two stages ahead (three A buffers) and decode the
-//    next stage's ternary weights from the packed bytes (copied into LDS by DMA two blocks
-//    ahead) into fp16 LDS tiles (two B buffers).  No fp16 weight copy ever touches HBM.
-//  * Decode: a group is 4 consecutive k of one row from the 4 bytes of one packed dword
-//    and one base-3 digit; the bytes go to 16-bit lanes (b0,b1) and (b2,b3), the digit is
-//    ((b * 3^n) mod 256) * 3 >> 8 with packed 16-bit multiplies, and v_perm_b32 picks the
-//    fp16 value -d, 0 or +d.
-//    A producer lane decodes half of one weight row (8 of its 16 groups per stage).
-//  * LDS rows are 64 halves (128 B) of 8 chunks of 16 B; chunk c of row r is stored at
-//    c ^ ((r >> 1) & 7).
-//  * Workgroups are numbered so that the ones on one XCD (dispatched round robin) share
-//    row tiles, and with them the A rows in that XCD's L2.
+// Design (MI355X-first; the reference expands every matrix to a 178 MB fp16 stage first): the
+// skeleton of gemm_reg.h with the PTQ1_0 decode below.  No fp16 weight copy exists, in HBM or in
+// LDS: a lane turns the packed bytes of its own column into the MFMA's B registers.
+//
+// What bounds it (K = 5120, N = 17408; before: 256 x 128 tiles whose producer waves wrote decoded
+// weights into LDS):
+//  * Many rows: power.  At 7300 rows every CU runs 256 x 256 tiles and the clock falls to 1.7 - 1.9
+//    of 2.4 GHz, so instructions and LDS bytes per MFMA count, not their latency: one wave per
+//    SIMD with 256 x 64 of C (2.7 vector instructions and half an LDS fragment read per MFMA)
+//    1337 -> 1100 us (1.18 PFLOP/s); a plain fp16 library product of the shape takes 1150.
+//    Two waves per SIMD of 128 x 64: 1118; of 128 x 32: 1220.
+//  * A hundred to a few hundred rows: vector instructions and MFMAs of the two waves of a SIMD
+//    overlap only in part (the stage barrier keeps them in step): 128 x 256 tiles, 200 rows
+//    80 -> 61 us.
+//  * Up to 64 rows: the decode (about 2.5 vector instructions per weight, each weight once per
+//    launch) and the fixed 3 us to the first MFMA; short tiles instead of rows of padding: 41
+//    rows 78 -> 28 us, 28 rows 78 -> 24 us.
+// Measured and not kept: trits from a conflict-free LDS table (half the vector instructions,
+// as many LDS cycles more: equal at 41 rows, 1.2x slower at 7300); waves of a SIMD in opposite
+// decode / multiply phases (1.1 - 1.3x slower: two barriers a unit); fragments read three or
+// seven steps ahead (equal).
 #include "common.h"
 #include "launch.h"
 
-#include <mutex>
-#include "gemm_tile.h"
-
 #include <algorithm>
 #include <type_traits>
+
+#include "gemm_reg.h"
 
 namespace kata {
 
 namespace {
 
-using namespace gemm;
-constexpr int kWStage = BN * 32;    // staged packed bytes of one block of the tile rows, 32 B per row
-constexpr int kLdsBytes = kTileBytes + 2 * kWStage;
-
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-
-// fp16 of (digit_n(b) - 1) * d for bytes in 16-bit lanes (b_lo, b_hi); lo = (-d, 0),
-// hi = (+d, +d) as fp16 bit pairs.  Returns the two halves as one dword.
-__device__ inline uint32_t decode_pair(u16x2 b, uint32_t p3n, uint32_t lo, uint32_t hi) {
-    u16x2 m = b * __builtin_bit_cast(u16x2, p3n);
-    m &= (u16x2){0xff, 0xff};
-    const u16x2 dg = (m * (u16x2){3, 3}) >> (u16x2){8, 8};
-    const u16x2 sel = dg * (u16x2){0x0202, 0x0202} + (u16x2){0x0100, 0x0100};
-    return __builtin_amdgcn_perm(hi, lo, __builtin_bit_cast(uint32_t, sel));
-}
-
-// group: bytes (b0, b1, b2, b3) of w -> 4 fp16 in that order as two dwords, digit n of
-// b0, b1 by the multipliers p3lo and of b2, b3 by p3hi; the bytes go to 16-bit lanes
-// (b0, b1) and (b2, b3) (v_perm selector 0x0c is a zero byte)
-__device__ inline uint2 group_vals(uint32_t w, uint32_t p3lo, uint32_t p3hi, uint32_t lo, uint32_t hi) {
-    const u16x2 e = __builtin_bit_cast(u16x2, __builtin_amdgcn_perm(0u, w, 0x0c010c00u));
-    const u16x2 o = __builtin_bit_cast(u16x2, __builtin_amdgcn_perm(0u, w, 0x0c030c02u));
-    return make_uint2(decode_pair(e, p3lo, lo, hi), decode_pair(o, p3hi, lo, hi));
-}
-__device__ inline uint2 group_vals(uint32_t w, uint32_t p3n, uint32_t lo, uint32_t hi) {
-    return group_vals(w, p3n, p3n, lo, hi);
-}
+using rg::u16x2;
 
 __host__ __device__ constexpr uint32_t p3x2(int n) {
     return n == 0 ? 0x00010001u : n == 1 ? 0x00030003u : n == 2 ? 0x00090009u : n == 3 ? 0x001b001bu : 0x00510051u;
 }
+// the bytes (b0, b1) / (b2, b3) of w in 16-bit lanes (v_perm selector 0x0c is a zero byte)
+__device__ inline u16x2 bytes01(uint32_t w) { return __builtin_bit_cast(u16x2, __builtin_amdgcn_perm(0u, w, 0x0c010c00u)); }
+__device__ inline u16x2 bytes23(uint32_t w) { return __builtin_bit_cast(u16x2, __builtin_amdgcn_perm(0u, w, 0x0c030c02u)); }
 
-// Decode groups of a stage (e = element of the block, dword j = bytes 4j..4j+3, stage
-// k = e - 64h; each group covers 4 consecutive k):
-//   h=0: dword i, digit n at k = 16n + 4i                        (i, n = 0..3)
-//   h=1: dword i digit 4 at k = 4i; dword 4+i digit n at k = 16 + 4i + 8n (n = 0..4);
-//        qh bytes (qh0, qh1, qh0, qh1) at digits (a, a, a+1, a+1) at k = 56 (a = 0) and 60 (a = 2)
-// Producer half-rows (half q of the row): a 16-byte LDS chunk holds two groups:
-//   h=0: chunk 2n + q = dwords 2q, 2q+1 at digit n (n = 0..3)
-//   h=1: q=0: chunk 0 = digit 4 of dwords 0,1; chunks 2,3,4 = digits 0,1,2 of dwords 4,5
-//        q=1: chunk 1 = digit 4 of dwords 2,3; chunks 5,6 = digits 3,4 of dwords 4,5;
-//             chunk 7 = the two qh groups
-template <bool C_F16>
-__global__ __launch_bounds__(512) void k_gemm_ptq1_f16(const _Float16* __restrict__ A, int lda,
-                                                       const uint8_t* __restrict__ W, void* __restrict__ C,
-                                                       int ldc, float* __restrict__ ws, int M, int K, int N,
-                                                       GemmJobs J) {
-    extern __shared__ __align__(16) uint8_t smem[];
-    auto Bs = [&](int buf) { return tile_b(smem, buf); };
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nbk = K >> 7;
-    int job, tile, kb0, nb;
-    gemm_job(J, nbk, job, tile, kb0, nb);
-    const int m0 = (tile / J.G) * BM;
-    const int n0 = (tile % J.G) * BN;
-    const int R = min(BN, N - n0);              // columns of this tile
-    const int nst = 2 * nb;                      // stages
-    const uint32_t row_bytes = (uint32_t)nbk * kBlockBytes;
-    A += (size_t)kb0 * 128;
-    auto barrier = [&]() { barrier_lds(); };
-
-    if (wave < 4) {
-        consume<C_F16>(smem, wave, lane, nst, job, J, ws, C, ldc, M, m0, n0, R);
-        return;
+// PTQ1_0 weights as B operand registers.  Lane half lh of column c takes chunk 2 kk + lh (8
+// consecutive k) of every 16-k step kk of a block: for kk < 5 digit kk of qs bytes 8 lh .. 8 lh
+// + 7; for kk = 5, 6 digit 2 (kk - 5) + lh of bytes 16..23; for kk = 7 digit 4 of those (lh = 0)
+// or the qh bytes, digit j for pair j (lh = 1).
+struct Ptq1F16 {
+    static constexpr int GROUP = 2;               // blocks per copied group: 56 bytes of a row
+    template <class C>
+    static constexpr int copies() {
+        static_assert(C::BN * 4 % C::THREADS == 0, "whole weight copies per thread");
+        return C::BN * 4 / C::THREADS;
     }
+    template <class C>
+    static constexpr int slot_bytes() { return C::BN * 64; }
 
-    // ================= producers =================
-    const int pw = wave - 4;
-    auto issue_a = [&](int st) { gemm::issue_a(smem, pw, lane, A, lda, M, m0, st, nst); };
-    // ---- weights: lane `lane` of producer pw decodes half q = pw & 1 of tile row
-    // 64 (pw >> 1) + lane (q wave-uniform: no divergence).  The packed bytes of a block of
-    // the tile's rows are copied into LDS by DMA (two 16-byte pieces per row, bytes 0..15
-    // and 12..27, so no copy reads past the row's block), two blocks ahead; a lane reads
-    // its dwords back when it starts the block.  Staging slot layout [piece][BN rows][16 B]:
-    // producer pw copies piece pw & 1 of rows 64 (pw >> 1) .. +63.
-    const int wrow = 64 * (pw >> 1) + lane, q = pw & 1;
-    const bool wactive = wrow < R;
-    uint8_t* Ws = smem + kABuf * BM * ROWB + 2 * BN * ROWB;      // [2 slots][2][BN][16 B]
-    const uint8_t* wsrc = W + (size_t)min(n0 + min(wrow, R - 1), N - 1) * row_bytes + (size_t)kb0 * kBlockBytes + 12 * q;
-    auto issue_w = [&](int blk) {
-        dma16(wsrc + (size_t)min(blk, nb - 1) * kBlockBytes,
-              lds_addr(Ws + (blk & 1) * kWStage + q * (BN * 16) + (pw >> 1) * 1024));
-    };
-    uint32_t w_cur[5];
-    auto read_w = [&](int blk) {
-        const uint8_t* slot = Ws + (blk & 1) * kWStage;
-        const uint2 a = *(const uint2*)(slot + wrow * 16 + 8 * q);                  // dwords 2q, 2q+1
-        const uint4 c = *(const uint4*)(slot + BN * 16 + wrow * 16);               // bytes 12..27
-        w_cur[0] = a.x;
-        w_cur[1] = a.y;
-        w_cur[2] = c.y;                                                            // dword 4
-        w_cur[3] = c.z;                                                            // dword 5
-        w_cur[4] = c.w;                                                            // dword 6
-    };
-    auto decode_w = [&](auto h_c, int buf) {
-        constexpr int h = decltype(h_c)::value;
-        if (!wactive) return;
-        uint8_t* bt = Bs(buf);
-        const uint32_t dbits = w_cur[4] >> 16;
-        const uint32_t lo = dbits ^ 0x8000u, hi = dbits | (dbits << 16);
-        auto put = [&](int chunk, uint2 a, uint2 b) {
-            *(uint4*)(bt + swz(wrow, chunk)) = make_uint4(a.x, a.y, b.x, b.y);
-        };
-        if (h == 0) {
+    const uint8_t* wbase[4];                      // copy sources: per instruction a uniform row base
+    uint32_t wvo[4];                              // and this lane's offset (full group)
+    uint32_t wsingle;                             // added to it in a group of one block
+    uint32_t w_lds;
+    uint32_t rd;                                  // LDS address of this lane's row (tile 0) in slot 0
+    uint32_t o_own0, o_p1, o_own10, o_own11, o_p2, o_p3;
+    int lh, nblk;
+    uint32_t wn[2][5];                            // next block's words: own half, bytes 16..27
+    u16x2 m[2][4];                                // remainders of the digits taken so far
+    uint32_t w4[2], w5[2], w6[2];
+    v2h dd[2], S[2];
+
+    // Copies: the 56 bytes of a row's group are four 16-byte pieces at 0, 16, 32, 40 (a last
+    // group of one block: 0, 12), so no copy reads past the row; row r's piece p sits in slot
+    // p ^ ((r >> 2) & 3) of its 64 LDS bytes.
+    template <class C>
+    __device__ inline void init(const uint8_t* W, int nbk, int kb0, int nb, int n0, int N, int tid, int wave, int wc,
+                                int l32, int lh_, uint32_t Ws) {
+        const uint32_t row_bytes = (uint32_t)nbk * kBlockBytes;
+        constexpr int RPI = C::THREADS / 4;
+        lh = lh_;
+        nblk = nb;
 #pragma unroll
-            for (int n = 0; n < 4; n++)
-                put(2 * n + q, group_vals(w_cur[0], p3x2(n), lo, hi), group_vals(w_cur[1], p3x2(n), lo, hi));
-        } else if (q == 0) {
-            put(0, group_vals(w_cur[0], p3x2(4), lo, hi), group_vals(w_cur[1], p3x2(4), lo, hi));
-#pragma unroll
-            for (int n = 0; n < 3; n++)
-                put(2 + n, group_vals(w_cur[2], p3x2(n), lo, hi), group_vals(w_cur[3], p3x2(n), lo, hi));
-        } else {
-            put(1, group_vals(w_cur[0], p3x2(4), lo, hi), group_vals(w_cur[1], p3x2(4), lo, hi));
-#pragma unroll
-            for (int n = 3; n < 5; n++)
-                put(2 + n, group_vals(w_cur[2], p3x2(n), lo, hi), group_vals(w_cur[3], p3x2(n), lo, hi));
-            const uint32_t qh = __builtin_amdgcn_perm(0u, w_cur[4], 0x01000100u);
-            put(7, group_vals(qh, p3x2(0), p3x2(1), lo, hi), group_vals(qh, p3x2(2), p3x2(3), lo, hi));
+        for (int i = 0; i < copies<C>(); i++) {
+            const int r0 = min(n0 + i * RPI, N - 1), r = tid / 4;
+            const int p = (tid & 3) ^ (((i * RPI + r) >> 2) & 3);
+            wbase[i] = W + (size_t)r0 * row_bytes + (size_t)kb0 * kBlockBytes;
+            wvo[i] = (uint32_t)min(r, N - 1 - r0) * row_bytes + (p < 3 ? 16u * p : 40u);
         }
-    };
-    using I0 = std::integral_constant<int, 0>;
-    using I1 = std::integral_constant<int, 1>;
-    // Vector-memory order of a producer (all its loads are LDS copies, which the compiler
-    // cannot count, so the waits below do): before the barrier that releases stage s, A
-    // batch s (8 copies) must have landed while the copies issued after it may still be in
-    // flight; a block's weight copy (1) goes after the A batch of its slot.
-    // prologue: weight blocks 0 and 1, A stages 0 and 1
-    issue_w(0);
-    issue_w(1);
-    issue_a(0);
-    issue_a(1);
-    // blocks 0, 1 and batch 0; a row's two weight pieces come from two waves
-    __builtin_amdgcn_s_waitcnt((8 & 15) | ((8 >> 4) << 14) | (7 << 4) | (15 << 8));
-    barrier();
-    read_w(0);
-    decode_w(I0(), 0);
-    barrier();
-    for (int b = 0; b < nb; b++) {
-        // consumers on stage 2b; produce stage 2b+1 (h=1 of block b) into B buffer 1
-        issue_a(2 * b + 2);
-        decode_w(I1(), 1);
-        __builtin_amdgcn_s_waitcnt((8 & 15) | ((8 >> 4) << 14) | (7 << 4) | (15 << 8));    // batch 2b+1, block b+1
-        barrier();
-        // consumers on stage 2b+1; produce stage 2b+2 (h=0 of block b+1) into B buffer 0
-        if (b + 1 < nb) read_w(b + 1);
-        issue_a(2 * b + 3);
-        issue_w(b + 2);                          // into the staging slot block b freed
-        if (b + 1 < nb) decode_w(I0(), 0);
-        __builtin_amdgcn_s_waitcnt((9 & 15) | ((9 >> 4) << 14) | (7 << 4) | (15 << 8));    // batch 2b+2
-        barrier();
+        const int p = (tid & 3) ^ ((tid >> 4) & 3);
+        wsingle = p == 0 ? 0u : (uint32_t)(12 - (p < 3 ? 16 * p : 40));
+        w_lds = Ws + 1024u * wave;
+        rd = Ws + (wc * 32 * C::NT + l32) * 64;
+        const uint32_t f = (uint32_t)(l32 >> 2) & 3u;
+        o_own0 = (f << 4) + 8u * lh;
+        o_p1 = (1u ^ f) << 4;
+        o_p2 = ((2u ^ f) << 4) + 12u;
+        o_p3 = ((3u ^ f) << 4) + 8u;
+        o_own10 = lh ? ((2u ^ f) << 4) + 4u : ((1u ^ f) << 4) + 12u;
+        o_own11 = ((2u ^ f) << 4) + (lh ? 8u : 0u);
     }
+    template <class C>
+    __device__ inline void issue(int g, int slot) {
+        const uint32_t add = 2 * g + 1 == nblk ? wsingle : 0u;
+#pragma unroll
+        for (int i = 0; i < copies<C>(); i++)
+            rg::dma16(wbase[i] + (size_t)g * (2 * kBlockBytes), wvo[i] + add,
+                      w_lds + slot * slot_bytes<C>() + i * (C::THREADS * 16));
+    }
+    template <class C, int J>
+    __device__ inline void read(int g, int slot, int nb) {
+        const uint32_t p = rd + slot * slot_bytes<C>();
+        auto word = [](uint32_t a) { return rg::lds_ld<uint32_t>(a); };
+#pragma unroll
+        for (int t = 0; t < C::NT; t++) {
+            if constexpr (J == 0) {
+                const uint32_t q = p + o_p1 + (2 * g + 1 == nb ? 4u : 0u) + t * 2048;
+                const rg::u32x2 a = rg::lds_ld<rg::u32x2>(p + o_own0 + t * 2048);
+                wn[t][0] = a.x;
+                wn[t][1] = a.y;
+                wn[t][2] = word(q);
+                wn[t][3] = word(q + 4);
+                wn[t][4] = word(q + 8);
+            } else {
+                wn[t][0] = word(p + o_own10 + t * 2048);
+                wn[t][1] = word(p + o_own11 + t * 2048);
+                wn[t][2] = word(p + o_p2 + t * 2048);
+                wn[t][3] = word(p + o_p3 + t * 2048);
+                wn[t][4] = word(p + o_p3 + 4 + t * 2048);
+            }
+        }
+    }
+    // Unpack the block read ahead.  True if a scale of the wave's columns is not below 1 in
+    // magnitude (or not finite): the fast form of `value` needs d * 2^16 in fp16.
+    template <class C>
+    __device__ inline bool begin() {
+        bool big = false;
+#pragma unroll
+        for (int t = 0; t < C::NT; t++) {
+            m[t][0] = bytes01(wn[t][0]);
+            m[t][1] = bytes23(wn[t][0]);
+            m[t][2] = bytes01(wn[t][1]);
+            m[t][3] = bytes23(wn[t][1]);
+            w4[t] = wn[t][2];
+            w5[t] = wn[t][3];
+            w6[t] = wn[t][4];
+            const uint32_t d2 = __builtin_amdgcn_perm(0u, w6[t], 0x03020302u);
+            dd[t] = __builtin_bit_cast(v2h, d2);
+            const v2h k = {(_Float16)256.0f, (_Float16)256.0f};
+            S[t] = dd[t] * k * k;
+            big |= (d2 & 0x7fffu) >= 0x3c00u;
+        }
+        return __any(big);
+    }
+    // fp16 of (digit - 1) * d for X = 3 m in 16-bit lanes, digit = X >> 8.  The digit's bits are
+    // the subnormal digit * 2^-16, so one fma with d * 2^16 and -d is exact (4 vector
+    // instructions per pair with the remainder update); with a scale of 1 or more the
+    // value is picked by a byte permute.
+    template <bool BIG>
+    __device__ inline uint32_t value(u16x2 X, int t) {
+        if constexpr (BIG) {
+            const uint32_t db = __builtin_bit_cast(uint32_t, dd[t]);
+            const u16x2 sel = (X >> (u16x2){8, 8}) * (u16x2){0x0202, 0x0202} + (u16x2){0x0100, 0x0100};
+            return __builtin_amdgcn_perm(db, (db & 0xffffu) ^ 0x8000u, __builtin_bit_cast(uint32_t, sel));
+        } else {
+            const v2h dg = __builtin_bit_cast(v2h, X & (u16x2){0x300, 0x300});
+            return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(dg, S[t], -dd[t]));
+        }
+    }
+    // chunk of 16-k step kk of the block, column tile t; steps in order
+    template <int kk, bool BIG>
+    __device__ inline v8h chunk(int t) {
+        const u16x2 three = {3, 3}, lo8 = {0xff, 0xff};
+        uint32_t o[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            u16x2 X;
+            if constexpr (kk < 5) {
+                X = m[t][j] * three;
+                if constexpr (kk < 4) m[t][j] = X & lo8;
+            } else if constexpr (kk == 5) {
+                const u16x2 mul = __builtin_bit_cast(u16x2, lh ? p3x2(1) : p3x2(0));
+                const uint32_t w = j < 2 ? w4[t] : w5[t];
+                m[t][j] = ((j & 1 ? bytes23(w) : bytes01(w)) * mul) & lo8;
+                X = m[t][j] * three;
+            } else if constexpr (kk == 6) {
+                m[t][j] = (m[t][j] * (u16x2){9, 9}) & lo8;
+                X = m[t][j] * three;
+            } else {
+                const uint32_t src = lh ? __builtin_bit_cast(uint32_t, bytes01(w6[t])) : __builtin_bit_cast(uint32_t, m[t][j]);
+                const u16x2 mul = __builtin_bit_cast(u16x2, lh ? p3x2(j) : p3x2(2));
+                X = ((__builtin_bit_cast(u16x2, src) * mul) & lo8) * three;
+            }
+            o[j] = value<BIG>(X, t);
+        }
+        return __builtin_bit_cast(v8h, make_uint4(o[0], o[1], o[2], o[3]));
+    }
+};
+
+template <class C, class D>
+constexpr int lds_bytes() { return C::ABUF * C::ASTAGE + (C::DW + 1) * D::template slot_bytes<C>(); }
+
+template <class C, bool C_F16>
+__global__ __launch_bounds__(C::THREADS, C::WPE) void k_gemm_ptq1_f16(const _Float16* __restrict__ A, int lda, rg::Mats P,
+                                                                      float* __restrict__ ws, int M, int K, GemmJobs J) {
+    rg::run<C, Ptq1F16, C_F16>(A, lda, P, ws, M, K, J);
 }
+
+//               MT NT WR WC  KS DA DW waves per SIMD
+typedef rg::Cfg<8, 2, 1, 4, 64, 2, 1, 1> Cfg256;     // 256 x 256
+typedef rg::Cfg<4, 1, 1, 8, 64, 2, 1, 2> Cfg128;     // 128 x 256
+typedef rg::Cfg<2, 1, 1, 8, 128, 2, 2, 2> Cfg64;     // 64 x 256
+typedef rg::Cfg<1, 1, 1, 8, 128, 2, 2, 2> Cfg32;     // 32 x 256
+// us per 128-k block of a tile, fitted to 25..7300 rows of the five model shapes; the schedule
+// that they choose is within 5 % of the best of all (tile, split) pairs at most of them
+constexpr int kBN = 256;
+constexpr rg::Shape kShapes[4] = {{32, kBN, 1.04f, 1.04f}, {64, kBN, 1.15f, 1.15f}, {128, kBN, 1.42f, 2.05f}, {256, kBN, 2.85f, 3.5f}};
 
 }  // namespace
 
@@ -204,37 +227,102 @@ hipError_t gemm_device(bool need_ws, hipStream_t s, int* n_cu, float** ws) {
     *ws = nullptr;
     if (!need_ws) return hipSuccess;
     void* p = nullptr;
-    e = stream_buffer(kBufGemmPieces, (size_t)*n_cu * 256 * 128 * sizeof(float), s, &p);
+    e = stream_buffer(kBufGemmPieces, (size_t)*n_cu * rg::kPieceFloats * sizeof(float), s, &p);
     *ws = (float*)p;
     return e;
 }
 
-hipError_t launch_gemm_f16(const uint16_t* A, int lda, const uint8_t* W, void* C, int c_dtype, int ldc,
-                           int M, int K, int N, hipStream_t s) {
+namespace {
+
+template <class C>
+hipError_t launch_cfg(const _Float16* A, int lda, const rg::Mats& P, float* ws, int c_dtype, bool v4, int M, int K,
+                      const GemmJobs& J, hipStream_t s) {
+    constexpr int kLds = lds_bytes<C, Ptq1F16>();
+    static_assert(kLds <= 160 * 1024, "LDS");
     // the dynamic-LDS limit of both instantiations, raised once per process (a function-local
     // static: thread-safe initialisation)
     static const hipError_t attr = [] {
-        hipError_t e = hipFuncSetAttribute((const void*)k_gemm_ptq1_f16<true>, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+        hipError_t e = hipFuncSetAttribute((const void*)k_gemm_ptq1_f16<C, true>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
         if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void*)k_gemm_ptq1_f16<false>, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+            e = hipFuncSetAttribute((const void*)k_gemm_ptq1_f16<C, false>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
         return e;
     }();
     if (attr != hipSuccess) return attr;
+    if (c_dtype == 1)
+        hipLaunchKernelGGL((k_gemm_ptq1_f16<C, true>), dim3(J.n_jobs), dim3(C::THREADS), kLds, s, A, lda, P, ws, M, K, J);
+    else
+        hipLaunchKernelGGL((k_gemm_ptq1_f16<C, false>), dim3(J.n_jobs), dim3(C::THREADS), kLds, s, A, lda, P, ws, M, K, J);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    return rg::launch_pieces_sum<C::BM, C::BN>(ws, P, c_dtype, v4, M, J, s);
+}
+
+}  // namespace
+
+hipError_t launch_gemm_f16_multi(const uint16_t* A, int lda, int count, const uint8_t* const* W, void* const* C, int c_dtype,
+                                 const int* ldc, int M, int K, const int* N, hipStream_t s) {
+    if (count < 1 || count > rg::kMaxMats) return hipErrorInvalidValue;
+    // the copies' row offsets are 32-bit: rows further apart go one by one
+    if (lda > (1 << 24) && M > 1) {
+        for (int m = 0; m < M; m++) {
+            void* Cm[rg::kMaxMats];
+            for (int i = 0; i < count; i++) Cm[i] = (uint8_t*)C[i] + (size_t)m * ldc[i] * (c_dtype == 1 ? 2 : 4);
+            hipError_t e = launch_gemm_f16_multi(A + (size_t)m * lda, K, count, W, Cm, c_dtype, ldc, 1, K, N, s);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
     int n_cu = 0;
     float* ws = nullptr;
     hipError_t e = gemm_device(false, s, &n_cu, &ws);
     if (e != hipSuccess) return e;
-    const GemmJobs J = plan_gemm_jobs(M, N, K, BM, BN, n_cu);   // one workgroup per CU
-    if (J.n_jobs > J.n_full && (e = gemm_device(true, s, &n_cu, &ws)) != hipSuccess) return e;
-    if (c_dtype == 1)
-        hipLaunchKernelGGL(k_gemm_ptq1_f16<true>, dim3(J.n_jobs), dim3(512), kLdsBytes, s, (const _Float16*)A, lda, W,
-                           C, ldc, ws, M, K, N, J);
-    else
-        hipLaunchKernelGGL(k_gemm_ptq1_f16<false>, dim3(J.n_jobs), dim3(512), kLdsBytes, s, (const _Float16*)A, lda,
-                           W, C, ldc, ws, M, K, N, J);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    return launch_pieces_sum<BM, BN>(ws, C, c_dtype, ldc, M, N, J, s);
+    rg::Mats P{};
+    bool v4 = true;
+    int G = 0;
+    for (int i = 0; i < rg::kMaxMats; i++) {
+        P.g0[i] = i < count ? G : 0x7fffffff;
+        if (i >= count) continue;
+        P.W[i] = W[i];
+        P.C[i] = C[i];
+        P.N[i] = N[i];
+        P.ldc[i] = ldc[i];
+        G += (N[i] + kBN - 1) / kBN;
+        v4 &= N[i] % 4 == 0 && ldc[i] % 4 == 0 && ((uintptr_t)C[i] & 15) == 0;
+    }
+    P.g0[rg::kMaxMats] = 0x7fffffff;
+    auto choose = [&](bool pieces, int& k) {
+        rg::Plan best{};
+        for (int i = 0; i < 4; i++) {
+            const rg::Plan p = rg::plan(kShapes[i], M, G, K / 128, n_cu, pieces);
+            if (i == 0 || p.us < best.us) {
+                best = p;
+                k = i;
+            }
+        }
+        return best.J;
+    };
+    int k = 0;
+    GemmJobs J = choose(true, k);
+    if (J.n_jobs > J.n_full) {
+        e = gemm_device(true, s, &n_cu, &ws);
+        if (e != hipSuccess) {
+            // no workspace (the stream's first call is captured, or memory is short): whole tiles
+            (void)hipGetLastError();
+            J = choose(false, k);
+        }
+    }
+    const _Float16* Ah = (const _Float16*)A;
+    switch (k) {
+        case 0: return launch_cfg<Cfg32>(Ah, lda, P, ws, c_dtype, v4, M, K, J, s);
+        case 1: return launch_cfg<Cfg64>(Ah, lda, P, ws, c_dtype, v4, M, K, J, s);
+        case 2: return launch_cfg<Cfg128>(Ah, lda, P, ws, c_dtype, v4, M, K, J, s);
+        default: return launch_cfg<Cfg256>(Ah, lda, P, ws, c_dtype, v4, M, K, J, s);
+    }
+}
+
+hipError_t launch_gemm_f16(const uint16_t* A, int lda, const uint8_t* W, void* C, int c_dtype, int ldc,
+                           int M, int K, int N, hipStream_t s) {
+    return launch_gemm_f16_multi(A, lda, 1, &W, &C, c_dtype, &ldc, M, K, &N, s);
 }
 
 }  // namespace kata

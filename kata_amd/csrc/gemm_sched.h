@@ -48,7 +48,8 @@ __device__ inline void gemm_job(const GemmJobs& J, int nbk, int& job, int& tile,
     const int lo = job < J.n_full ? 0 : J.n_full;
     const int n = job < J.n_full ? J.n_full : J.n_jobs - J.n_full;
     const int i = job - lo;
-    if (n % 8 == 0 && lo % 8 == 0) job = lo + (i % 8) * (n / 8) + i / 8;
+    // (a bijection for any n: XCD x takes n / 8 jobs, one more for x < n % 8)
+    job = lo + (i % 8) * (n / 8) + min(i % 8, n % 8) + i / 8;
     if (job < J.n_full) {
         tile = job;
         kb0 = 0;

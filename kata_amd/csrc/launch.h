@@ -46,6 +46,9 @@ int gemv_q8_max_mats();
 // ---- prefill (gemm_f16.hip, gemm_i8.hip, expand.hip)
 hipError_t launch_gemm_f16(const uint16_t* A, int lda, const uint8_t* W, void* C, int c_dtype, int ldc,
                            int M, int K, int N, hipStream_t s);
+// the same for 1..4 matrices sharing A, one launch
+hipError_t launch_gemm_f16_multi(const uint16_t* A, int lda, int count, const uint8_t* const* W, void* const* C,
+                                 int c_dtype, const int* ldc, int M, int K, const int* N, hipStream_t s);
 hipError_t launch_gemm_q8(const uint16_t* A, int lda, const uint8_t* W, void* C, int c_dtype, int ldc, int M, int K,
                           int N, hipStream_t s);
 hipError_t launch_quant_rows(const uint16_t* X, int8_t* Q, float* SX, int M, int K, int ldS,

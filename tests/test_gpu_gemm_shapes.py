@@ -1,0 +1,108 @@
+"""The fp16 prefill GEMM over the sizes where its tile shapes and schedules change: rows at
+the edges of the 32, 64, 128 and 256 row tiles, columns around the 256 column tiles, odd and
+even numbers of 128-k blocks (the packed weights are copied two blocks at a time), K splits of
+all tiles and of the last round, scales of 1 and more (another decode form), several matrices in
+one launch, and rows too far apart for 32-bit offsets.
+
+Reference: float64 products of the expanded weights.  Bar: fp32 sums of K fp16 products err by
+about sqrt(K) 2^-24 of their scale, at most 8e-6 at K = 17408 (1e-5 as for the other shapes)."""
+import numpy as np
+import pytest
+import torch
+
+from kata_amd import ops
+from kata_amd.engine import Dispatch, dispatch_work_bytes
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+def _weights(dev, K, N, seed, big):
+    rng = np.random.default_rng(seed)
+    t = rng.integers(-1, 2, (N, K)).astype(np.int8)
+    d = np.abs(rng.normal(0, 0.02, (N, K // 128)))
+    if big:                                     # blocks at and above 1, tiny and zero scales
+        d[:, ::3] *= 5000.0
+        d[1::7] = 1.0
+        d[::5, 1::4] = 3e-7
+        d[::11] = 0.0
+    return torch.from_numpy(orc.pack(t, d.astype(np.float16))).to(dev)
+
+
+def _check(C, A, W, K, N):
+    ref = A.double() @ ops.expand_f16(W, K, N).double().t()
+    err = float((C.double() - ref).norm() / ref.norm())
+    assert err < 1e-5, err
+
+
+@pytest.mark.parametrize("big", [False, True])
+@pytest.mark.parametrize("M", [1, 31, 32, 33, 64, 65, 127, 129, 256, 257, 700])
+@pytest.mark.parametrize("K,N", [(128, 257), (384, 1000), (2176, 256), (5120, 255)])
+def test_tile_edges(dev, M, K, N, big):
+    W = _weights(dev, K, N, M + K + N, big)
+    A = torch.from_numpy(orc.synth_x(M, K, M + 5)).to(dev)
+    _check(ops.gemm_ptq1_f16(A, W, K, N), A, W, K, N)
+
+
+@pytest.mark.parametrize("M,K,N", [(1024, 1024, 17000), (4500, 640, 5000), (2000, 5120, 1024)])
+def test_schedules(dev, M, K, N):
+    """Whole rounds with a split rest, and every tile split, at sizes of the larger tiles."""
+    W = _weights(dev, K, N, M + K, False)
+    A = torch.from_numpy(orc.synth_x(M, K, M + 6)).to(dev)
+    C = ops.gemm_ptq1_f16(A, W, K, N)
+    _check(C, A, W, K, N)
+    assert torch.equal(ops.gemm_ptq1_f16(A, W, K, N, out_dtype=torch.float16), C.half())
+
+
+def test_strided_and_unaligned(dev):
+    """lda > K, an odd ldc > N, and a weight base at a 2-byte (not 4-byte) address."""
+    M, K, N = 70, 640, 301
+    W = _weights(dev, K, N, 9, False)
+    buf = torch.zeros(W.numel() + 2, dtype=torch.uint8, device=dev)
+    buf[2:] = W.reshape(-1)
+    A = torch.from_numpy(orc.synth_x(M, K + 8, 10)).to(dev)
+    out = torch.full((M, N + 6), 7.0, device=dev)
+    ops.gemm_ptq1_f16(A, buf[2:], K, N, out=out)
+    _check(out[:, :N], A[:, :K], W, K, N)
+    assert bool((out[:, N:] == 7.0).all())
+
+
+@pytest.mark.parametrize("M", [30, 200])
+def test_matrices_of_one_launch(dev, M):
+    """The dispatcher's prefill form runs the matrices that share an input as one launch: ragged
+    widths, each against its own product; an int8 one among them goes its own way."""
+    H = 1024
+    Ns, names = (300, 1024, 129, 2050), ("qkv", "wq", "wk", "z")
+    Ws = [_weights(dev, H, N, 20 + i, False) for i, N in enumerate(Ns)]
+    offs = np.cumsum([0] + [W.numel() for W in Ws])
+    d = Dispatch(torch.cat([W.reshape(-1) for W in Ws]))
+    x = torch.from_numpy(orc.synth_x(M, H, 30)).to(dev).float()
+    gs = torch.ones(H, device=dev)
+    work = torch.empty(dispatch_work_bytes("prefill", H, M), dtype=torch.uint8, device=dev)
+    for i8 in ("none", "wq"):
+        d.set_i8(i8)
+        outs = d.sub_in("prefill", [(int(offs[i]), Ns[i], names[i]) for i in range(4)], x, None, gs, work=work)
+        h = work[:2 * M * H].view(torch.float16).view(M, H)
+        for W, N, nm, C in zip(Ws, Ns, names, outs):
+            if nm == i8:
+                Q, SX = ops.quant_rows(h.contiguous())
+                assert torch.equal(C, ops.gemm_ptq1_i8(Q, SX, W, H, N))
+            else:
+                _check(C, h, W, H, N)
+
+
+def test_first_call_captured(dev):
+    """A stream's first GEMM may be captured: without the workspace no tile is split."""
+    M, K, N = 40, 2048, 1024
+    W = _weights(dev, K, N, 40, False)
+    A = torch.from_numpy(orc.synth_x(M, K, 41)).to(dev)
+    C = torch.empty((M, N), device=dev)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=torch.cuda.Stream(dev)):
+        ops.gemm_ptq1_f16(A, W, K, N, out=C)
+    for _ in range(3):
+        C.fill_(float("nan"))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        _check(C, A, W, K, N)
