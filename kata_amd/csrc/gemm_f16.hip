@@ -52,6 +52,8 @@ __device__ inline u16x2 bytes23(uint32_t w) { return __builtin_bit_cast(u16x2, _
 // + 7; for kk = 5, 6 digit 2 (kk - 5) + lh of bytes 16..23; for kk = 7 digit 4 of those (lh = 0)
 // or the qh bytes, digit j for pair j (lh = 1).
 struct Ptq1F16 {
+    static constexpr bool TWO_FORMS = true;
+    static constexpr int kBlockB = kBlockBytes;   // bytes of 128 k of a row
     static constexpr int GROUP = 2;               // blocks per copied group: 56 bytes of a row
     template <class C>
     static constexpr int copies() {
@@ -103,10 +105,10 @@ struct Ptq1F16 {
         o_own11 = ((2u ^ f) << 4) + (lh ? 8u : 0u);
     }
     template <class C>
-    __device__ inline void issue(int g, int slot) {
+    __device__ inline void issue(int g, int slot, int i0, int i1) {
         const uint32_t add = 2 * g + 1 == nblk ? wsingle : 0u;
 #pragma unroll
-        for (int i = 0; i < copies<C>(); i++)
+        for (int i = i0; i < i1; i++)
             rg::dma16(wbase[i] + (size_t)g * (2 * kBlockBytes), wvo[i] + add,
                       w_lds + slot * slot_bytes<C>() + i * (C::THREADS * 16));
     }
@@ -133,6 +135,8 @@ struct Ptq1F16 {
             }
         }
     }
+    template <class C, int kb>
+    __device__ inline void look(int) {}
     // Unpack the block read ahead.  True if a scale of the wave's columns is not below 1 in
     // magnitude (or not finite): the fast form of `value` needs d * 2^16 in fp16.
     template <class C>
@@ -200,24 +204,18 @@ struct Ptq1F16 {
     }
 };
 
-template <class C, class D>
-constexpr int lds_bytes() { return C::ABUF * C::ASTAGE + (C::DW + 1) * D::template slot_bytes<C>(); }
-
-template <class C, bool C_F16>
-__global__ __launch_bounds__(C::THREADS, C::WPE) void k_gemm_ptq1_f16(const _Float16* __restrict__ A, int lda, rg::Mats P,
-                                                                      float* __restrict__ ws, int M, int K, GemmJobs J) {
-    rg::run<C, Ptq1F16, C_F16>(A, lda, P, ws, M, K, J);
-}
-
 //               MT NT WR WC  KS DA DW waves per SIMD
 typedef rg::Cfg<8, 2, 1, 4, 64, 2, 1, 1> Cfg256;     // 256 x 256
 typedef rg::Cfg<4, 1, 1, 8, 64, 2, 1, 2> Cfg128;     // 128 x 256
 typedef rg::Cfg<2, 1, 1, 8, 128, 2, 2, 2> Cfg64;     // 64 x 256
 typedef rg::Cfg<1, 1, 1, 8, 128, 2, 2, 2> Cfg32;     // 32 x 256
 // us per 128-k block of a tile, fitted to 25..7300 rows of the five model shapes; the schedule
-// that they choose is within 5 % of the best of all (tile, split) pairs at most of them
+// that they choose is within 5 % of the best of all (tile, split) pairs at most of them.  Pieces
+// of fewer than 8 blocks gain little (41 rows, 6144 -> 5120: 18.3 us in 6 pieces, 16.8 in 12), and
+// 8 keeps that product's row sums in the pieces of 256 x 128 tiles: behind three layers of fp16
+// rounding an output then differs by 2.9e-4 from those, not 4.9e-4.
 constexpr int kBN = 256;
-constexpr rg::Shape kShapes[4] = {{32, kBN, 1.04f, 1.04f}, {64, kBN, 1.15f, 1.15f}, {128, kBN, 1.42f, 2.05f}, {256, kBN, 2.85f, 3.5f}};
+constexpr rg::Shape kShapes[4] = {{32, kBN, 1.04f, 1.04f, 8}, {64, kBN, 1.15f, 1.15f, 8}, {128, kBN, 1.42f, 2.05f, 8}, {256, kBN, 2.85f, 3.5f, 8}};
 
 }  // namespace
 
@@ -232,92 +230,9 @@ hipError_t gemm_device(bool need_ws, hipStream_t s, int* n_cu, float** ws) {
     return e;
 }
 
-namespace {
-
-template <class C>
-hipError_t launch_cfg(const _Float16* A, int lda, const rg::Mats& P, float* ws, int c_dtype, bool v4, int M, int K,
-                      const GemmJobs& J, hipStream_t s) {
-    constexpr int kLds = lds_bytes<C, Ptq1F16>();
-    static_assert(kLds <= 160 * 1024, "LDS");
-    // the dynamic-LDS limit of both instantiations, raised once per process (a function-local
-    // static: thread-safe initialisation)
-    static const hipError_t attr = [] {
-        hipError_t e = hipFuncSetAttribute((const void*)k_gemm_ptq1_f16<C, true>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void*)k_gemm_ptq1_f16<C, false>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
-        return e;
-    }();
-    if (attr != hipSuccess) return attr;
-    if (c_dtype == 1)
-        hipLaunchKernelGGL((k_gemm_ptq1_f16<C, true>), dim3(J.n_jobs), dim3(C::THREADS), kLds, s, A, lda, P, ws, M, K, J);
-    else
-        hipLaunchKernelGGL((k_gemm_ptq1_f16<C, false>), dim3(J.n_jobs), dim3(C::THREADS), kLds, s, A, lda, P, ws, M, K, J);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    return rg::launch_pieces_sum<C::BM, C::BN>(ws, P, c_dtype, v4, M, J, s);
-}
-
-}  // namespace
-
 hipError_t launch_gemm_f16_multi(const uint16_t* A, int lda, int count, const uint8_t* const* W, void* const* C, int c_dtype,
                                  const int* ldc, int M, int K, const int* N, hipStream_t s) {
-    if (count < 1 || count > rg::kMaxMats) return hipErrorInvalidValue;
-    // the copies' row offsets are 32-bit: rows further apart go one by one
-    if (lda > (1 << 24) && M > 1) {
-        for (int m = 0; m < M; m++) {
-            void* Cm[rg::kMaxMats];
-            for (int i = 0; i < count; i++) Cm[i] = (uint8_t*)C[i] + (size_t)m * ldc[i] * (c_dtype == 1 ? 2 : 4);
-            hipError_t e = launch_gemm_f16_multi(A + (size_t)m * lda, K, count, W, Cm, c_dtype, ldc, 1, K, N, s);
-            if (e != hipSuccess) return e;
-        }
-        return hipSuccess;
-    }
-    int n_cu = 0;
-    float* ws = nullptr;
-    hipError_t e = gemm_device(false, s, &n_cu, &ws);
-    if (e != hipSuccess) return e;
-    rg::Mats P{};
-    bool v4 = true;
-    int G = 0;
-    for (int i = 0; i < rg::kMaxMats; i++) {
-        P.g0[i] = i < count ? G : 0x7fffffff;
-        if (i >= count) continue;
-        P.W[i] = W[i];
-        P.C[i] = C[i];
-        P.N[i] = N[i];
-        P.ldc[i] = ldc[i];
-        G += (N[i] + kBN - 1) / kBN;
-        v4 &= N[i] % 4 == 0 && ldc[i] % 4 == 0 && ((uintptr_t)C[i] & 15) == 0;
-    }
-    P.g0[rg::kMaxMats] = 0x7fffffff;
-    auto choose = [&](bool pieces, int& k) {
-        rg::Plan best{};
-        for (int i = 0; i < 4; i++) {
-            const rg::Plan p = rg::plan(kShapes[i], M, G, K / 128, n_cu, pieces);
-            if (i == 0 || p.us < best.us) {
-                best = p;
-                k = i;
-            }
-        }
-        return best.J;
-    };
-    int k = 0;
-    GemmJobs J = choose(true, k);
-    if (J.n_jobs > J.n_full) {
-        e = gemm_device(true, s, &n_cu, &ws);
-        if (e != hipSuccess) {
-            // no workspace (the stream's first call is captured, or memory is short): whole tiles
-            (void)hipGetLastError();
-            J = choose(false, k);
-        }
-    }
-    const _Float16* Ah = (const _Float16*)A;
-    switch (k) {
-        case 0: return launch_cfg<Cfg32>(Ah, lda, P, ws, c_dtype, v4, M, K, J, s);
-        case 1: return launch_cfg<Cfg64>(Ah, lda, P, ws, c_dtype, v4, M, K, J, s);
-        case 2: return launch_cfg<Cfg128>(Ah, lda, P, ws, c_dtype, v4, M, K, J, s);
-        default: return launch_cfg<Cfg256>(Ah, lda, P, ws, c_dtype, v4, M, K, J, s);
-    }
+    return rg::launch<Ptq1F16, Cfg32, Cfg64, Cfg128, Cfg256>(kShapes, (const _Float16*)A, lda, count, W, C, c_dtype, ldc, M, K, N, s);
 }
 
 hipError_t launch_gemm_f16(const uint16_t* A, int lda, const uint8_t* W, void* C, int c_dtype, int ldc,

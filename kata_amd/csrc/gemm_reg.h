@@ -15,6 +15,8 @@
 //    the end repeat the last stage or group).
 #pragma once
 #include <algorithm>
+#include <array>
+#include <cstdlib>
 #include <utility>
 
 #include "common.h"
@@ -93,7 +95,10 @@ __device__ inline void barrier_lds() {
     asm volatile("" ::: "memory");
 }
 
-// One job.  D: the weight format (see Ptq1F16 in gemm_f16.hip).
+// One job.  D: the weight format (Ptq1F16 in gemm_f16.hip, Q8F16 in gemm_q8.hip): its copies, and
+// chunk<kk, general>(t), the B operand of 16-k step kk and column tile t, steps in order.  A format
+// reads its words from LDS one block ahead (read, unpacked by begin) or two steps ahead (look).
+// TWO_FORMS: begin's result selects the general form of the chunks.
 template <class C, class D, bool C_F16>
 __device__ inline void run(const _Float16* __restrict__ A, int lda, const Mats& P, float* __restrict__ ws, int M,
                            int K, const GemmJobs& J) {
@@ -135,7 +140,11 @@ __device__ inline void run(const _Float16* __restrict__ A, int lda, const Mats& 
     };
     D dec;
     dec.template init<C>(W, nbk, kb0, nb, n0, N, tid, wave, wc, l32, lh, Ws);
-    auto issue_w = [&](int g) { dec.template issue<C>(min(g, ng - 1), g % (DW + 1)); };
+    auto issue_w = [&](int g, int i0, int i1) { dec.template issue<C>(min(g, ng - 1), g % (DW + 1), i0, i1); };
+    // A group's weight copies are issued in its DW-th last group's first stage, or, where they
+    // still land in time, over all of that group's stages
+    constexpr bool SPREAD = (DW - 1) * SPG >= DA;
+    auto w0 = [](int sp) constexpr { return SPREAD ? sp * NW / SPG : sp == 0 ? 0 : NW; };
 
     v16f acc[MT][NT];
 #pragma unroll
@@ -149,14 +158,15 @@ __device__ inline void run(const _Float16* __restrict__ A, int lda, const Mats& 
     constexpr int PRE = DA > DW * SPG ? DA : DW * SPG;
     unroll<PRE>([&](auto ic) {
         constexpr int j = decltype(ic)::value - PRE;
-        if constexpr (j % SPG == 0 && j >= -DW * SPG) issue_w(j / SPG + DW);
+        constexpr int sp = ((j % SPG) + SPG) % SPG;
+        if constexpr (j >= -DW * SPG) issue_w((j - sp) / SPG + DW, w0(sp), w0(sp + 1));
         if constexpr (j >= -DA) issue_a(j + DA, (j + DA) % ABUF, 0, NA);
     });
     // copies that may still fly when stage sp (of its group) starts: those issued after A(s),
     // which is issued over stage s - DA, after that stage's weight copies
-    auto vm_of = [](int sp) constexpr {
+    auto vm_of = [w0](int sp) constexpr {
         int n = (DA - 1) * NA;
-        for (int j = sp - DA + 1; j < sp; j++) n += (j % SPG == 0) ? NW : 0;
+        for (int j = sp - DA + 1; j < sp; j++) n += w0((j + SPG) % SPG + 1) - w0((j + SPG) % SPG);
         return n;
     };
     // A fragment addresses: row l32 of each 32-row tile, chunk 2 kk + lh
@@ -179,10 +189,12 @@ __device__ inline void run(const _Float16* __restrict__ A, int lda, const Mats& 
     // first fragments and chunk
     next_stage(std::integral_constant<int, 0>{});
     dec.template read<C, 0>(0, 0, nb);
+    dec.template look<C, 6>(-1);
     frags(std::integral_constant<int, 0>{}, af[0]);
     bool big = dec.template begin<C>();
 #pragma unroll
     for (int t = 0; t < NT; t++) bf[0][t] = dec.template chunk<0, true>(t);
+    dec.template look<C, 7>(-1);
     // Step kk of a block: the fragments and the decode of step kk + 1 run beside the MFMAs of
     // step kk.  A block's chunk 0 is decoded before its scales choose the form of the others.
     auto do_block = [&](auto jc, int g, auto bigc) {
@@ -209,6 +221,7 @@ __device__ inline void run(const _Float16* __restrict__ A, int lda, const Mats& 
                         else
                             dec.template read<C, 0>(g + 1, (g + 1) % (DW + 1), nb);
                     }
+                    dec.template look<C, kb>(g);
                 }
                 if constexpr (kb < 7) bf[nxt][t] = dec.template chunk<(kb + 1) % 8, BIG>(t);
                 else bf[nxt][t] = dec.template chunk<0, true>(t);
@@ -222,7 +235,7 @@ __device__ inline void run(const _Float16* __restrict__ A, int lda, const Mats& 
                     __builtin_amdgcn_sched_group_barrier(0x2, 5, 0);
                 }
                 __builtin_amdgcn_sched_barrier(0);
-                if constexpr (kk == 0 && sp == 0 && t == 0) issue_w(g + DW);
+                if constexpr (kk == 0 && t == 0) issue_w(g + DW, w0(sp), w0(sp + 1));
                 // the copies of stage s + DA, spread over the steps before the stage's last (whose
                 // barrier comes first)
                 if constexpr (kk + 1 < NKK) {
@@ -250,7 +263,8 @@ __device__ inline void run(const _Float16* __restrict__ A, int lda, const Mats& 
         b0 = nb;
     };
     blocks(std::false_type{});
-    if (__builtin_expect(b0 < nb, 0)) blocks(std::true_type{});
+    if constexpr (D::TWO_FORMS)
+        if (__builtin_expect(b0 < nb, 0)) blocks(std::true_type{});
     wait_vm<0>();                                             // the repeated copies, before the LDS is given back
 
     // store: lane holds D[8(q/4) + 4 lh + q%4][l32] of each 32 x 32 tile
@@ -348,16 +362,13 @@ inline hipError_t launch_pieces_sum(const float* ws, const Mats& P, int c_dtype,
 struct Shape {
     int bm, bn;
     float t_alone, t_full;
+    int min_blocks;      // of a piece where every tile is split
 };
 struct Plan {
     GemmJobs J;
     float us;
 };
 constexpr int kPieceFloats = 2 * 256 * 128;               // workspace floats per CU
-// Blocks of a piece where every tile is split.  Fewer gain little (41 rows, 6144 -> 5120: 18.3 us
-// in 6 pieces, 16.8 in 12), and 8 keeps that product's row sums in the pieces of 256 x 128 tiles:
-// behind three layers of fp16 rounding an output then differs by 2.9e-4 from those, not 4.9e-4.
-constexpr int kMinPieceBlocks = 8;
 // The cheapest schedule of T = row tiles x column groups tiles on n_cu workgroups: whole tiles
 // for the full rounds and the rest split S ways, or every tile split; a split costs the
 // pieces' way through memory and back (4 TB/s) and a launch (4 us); a round starts in 3 us.
@@ -372,7 +383,7 @@ inline Plan plan(const Shape& c, int M, int G, int nbk, int n_cu, bool pieces) {
     Plan best{{G, (int)T, 1, (int)T}, (float)part(T, nbk)};
     if (!pieces) return best;
     for (long rem : {T % n_cu, T}) {
-        for (int S = 2; rem && S <= kMaxPieces && S * (rem == T ? kMinPieceBlocks : 1) <= nbk; S++) {
+        for (int S = 2; rem && S <= kMaxPieces && S * (rem == T ? c.min_blocks : 1) <= nbk; S++) {
             if ((double)rem * S * c.bm * c.bn > (double)n_cu * kPieceFloats) break;
             const double us = (T > rem ? part(T - rem, nbk) : 0.0) + part(rem * S, (nbk + S - 1) / S) + 4.0 +
                               rem * S * rows * c.bn * 8.0 / 4e6;
@@ -380,6 +391,114 @@ inline Plan plan(const Shape& c, int M, int G, int nbk, int n_cu, bool pieces) {
         }
     }
     return best;
+}
+
+template <class D, class C, bool C_F16>
+__global__ __launch_bounds__(C::THREADS, C::WPE) void k_gemm(const _Float16* __restrict__ A, int lda, Mats P,
+                                                             float* __restrict__ ws, int M, int K, GemmJobs J) {
+    run<C, D, C_F16>(A, lda, P, ws, M, K, J);
+}
+
+template <class D, class C>
+hipError_t launch_cfg(const _Float16* A, int lda, const Mats& P, float* ws, int c_dtype, bool v4, int M, int K,
+                      const GemmJobs& J, hipStream_t s) {
+    static constexpr int kLds = C::ABUF * C::ASTAGE + (C::DW + 1) * D::template slot_bytes<C>();
+    static_assert(kLds <= 160 * 1024, "LDS");
+    // the dynamic-LDS limit of both instantiations, raised once per process (a function-local
+    // static: thread-safe initialisation)
+    static const hipError_t attr = [] {
+        hipError_t e = hipFuncSetAttribute((const void*)k_gemm<D, C, true>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute((const void*)k_gemm<D, C, false>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+        return e;
+    }();
+    if (attr != hipSuccess) return attr;
+    if (c_dtype == 1)
+        hipLaunchKernelGGL((k_gemm<D, C, true>), dim3(J.n_jobs), dim3(C::THREADS), kLds, s, A, lda, P, ws, M, K, J);
+    else
+        hipLaunchKernelGGL((k_gemm<D, C, false>), dim3(J.n_jobs), dim3(C::THREADS), kLds, s, A, lda, P, ws, M, K, J);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    return launch_pieces_sum<C::BM, C::BN>(ws, P, c_dtype, v4, M, J, s);
+}
+
+// C[i] = A W[i]^T for 1..4 matrices of weight format D, on the cheapest of the configurations
+// (all with the same column width) that `shapes` describes in the same order.
+template <class D, class... Cs>
+hipError_t launch(const Shape (&shapes)[sizeof...(Cs)], const _Float16* A, int lda, int count, const uint8_t* const* W, void* const* C,
+                  int c_dtype, const int* ldc, int M, int K, const int* N, hipStream_t s) {
+    constexpr int kShapes = sizeof...(Cs), BN = std::get<0>(std::array<int, kShapes>{Cs::BN...});
+    static_assert(((Cs::BN == BN) && ...), "one column width");
+    if (count < 1 || count > kMaxMats) return hipErrorInvalidValue;
+    // the copies' row offsets are 32-bit: rows further apart go one by one
+    if (lda > (1 << 24) && M > 1) {
+        for (int m = 0; m < M; m++) {
+            void* Cm[kMaxMats];
+            for (int i = 0; i < count; i++) Cm[i] = (uint8_t*)C[i] + (size_t)m * ldc[i] * (c_dtype == 1 ? 2 : 4);
+            hipError_t e = launch<D, Cs...>(shapes, A + (size_t)m * lda, K, count, W, Cm, c_dtype, ldc, 1, K, N, s);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
+    // and so are those of the weight rows of a tile: longer rows go a few at a time
+    const size_t row_bytes = (size_t)(K / 128) * D::kBlockB;
+    if (row_bytes > 0xffffffffu / BN) {
+        const int n = (int)std::max<size_t>(1, 0xffffffffu / row_bytes);
+        for (int i = 0; i < count; i++)
+            for (int n0 = 0; count > 1 || N[i] > n ? n0 < N[i] : false; n0 += n) {
+                const uint8_t* Wn = W[i] + (size_t)n0 * row_bytes;
+                void* Cn = (uint8_t*)C[i] + (size_t)n0 * (c_dtype == 1 ? 2 : 4);
+                const int Nn = std::min(n, N[i] - n0);
+                hipError_t e = launch<D, Cs...>(shapes, A, lda, 1, &Wn, &Cn, c_dtype, ldc + i, M, K, &Nn, s);
+                if (e != hipSuccess) return e;
+            }
+        if (count > 1 || N[0] > n) return hipSuccess;
+    }
+    int n_cu = 0;
+    float* ws = nullptr;
+    hipError_t e = gemm_device(false, s, &n_cu, &ws);
+    if (e != hipSuccess) return e;
+    Mats P{};
+    bool v4 = true;
+    int G = 0;
+    for (int i = 0; i < kMaxMats; i++) {
+        P.g0[i] = i < count ? G : 0x7fffffff;
+        if (i >= count) continue;
+        P.W[i] = W[i];
+        P.C[i] = C[i];
+        P.N[i] = N[i];
+        P.ldc[i] = ldc[i];
+        G += (N[i] + BN - 1) / BN;
+        v4 &= N[i] % 4 == 0 && ldc[i] % 4 == 0 && ((uintptr_t)C[i] & 15) == 0;
+    }
+    P.g0[kMaxMats] = 0x7fffffff;
+    int k = 0;
+    auto choose = [&](bool pieces) {
+        Plan best{};
+        for (int i = 0; i < kShapes; i++) {
+            const Plan p = plan(shapes[i], M, G, K / 128, n_cu, pieces);
+            if (i == 0 || p.us < best.us) {
+                best = p;
+                k = i;
+            }
+        }
+        return best.J;
+    };
+    GemmJobs J = choose(true);
+#ifdef TUNE
+    if (const char* q = getenv("KBM")) {
+        k = atoi(q); J = plan(shapes[k], M, G, K / 128, n_cu, true).J;
+        if (const char* q2 = getenv("KS")) { const int T = (M + shapes[k].bm - 1) / shapes[k].bm * G, S = atoi(q2); if (S > K / 128 || S > 16 || (double)T * S * shapes[k].bm * shapes[k].bn > (double)n_cu * kPieceFloats) return hipErrorInvalidValue; J = S > 1 ? GemmJobs{G, 0, S, T * S} : GemmJobs{G, T, 1, T}; }
+    }
+#endif
+    if (J.n_jobs > J.n_full && gemm_device(true, s, &n_cu, &ws) != hipSuccess) {
+        // no workspace (the stream's first call is captured, or memory is short): whole tiles
+        (void)hipGetLastError();
+        J = choose(false);
+    }
+    int i = 0;
+    ((i++ == k ? (void)(e = launch_cfg<D, Cs>(A, lda, P, ws, c_dtype, v4, M, K, J, s)) : (void)0), ...);
+    return e;
 }
 
 }  // namespace rg

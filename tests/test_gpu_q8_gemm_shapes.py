@@ -1,0 +1,28 @@
+"""The Q8_0 prefill GEMM over the sizes where its tile shapes and schedules change: rows at the
+edges of the 64, 128 and 256 row tiles, columns around the 256 column tiles, one to many 128-k
+blocks, K splits, and the last rows of the matrix at the end of an allocation.
+
+Reference: float64 products of the expanded weights.  Bar: 1e-5 relative L2 (fp32 sums of K fp16
+products err by about sqrt(K) 2^-24 of their scale)."""
+import numpy as np
+import pytest
+import torch
+
+from kata_amd import ops
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M", [1, 63, 64, 65, 128, 129, 256, 300, 900])
+@pytest.mark.parametrize("K,N", [(128, 3), (256, 257), (640, 255), (5120, 1024)])
+def test_tile_edges(dev, M, K, N):
+    W_np, q, d = orc.synth_q8(N, K, M + K + N)
+    A = torch.from_numpy(orc.synth_x(M, K, M + 1)).to(dev)
+    C = ops.gemm_q8_f16(A, torch.from_numpy(W_np).to(dev), K, N)
+    w = (torch.from_numpy(q).to(dev).double().view(N, K // 32, 32) *
+         torch.from_numpy(d.astype(np.float64)).to(dev)[:, :, None]).half().double().view(N, K)
+    ref = A.double() @ w.t()
+    err = float((C.double() - ref).norm() / ref.norm())
+    assert err < 1e-5, err
+    assert torch.equal(ops.gemm_q8_f16(A, torch.from_numpy(W_np).to(dev), K, N, out_dtype=torch.float16), C.half())
