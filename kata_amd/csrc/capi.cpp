@@ -649,10 +649,13 @@ int kata_dispatch_ffn_prefill(kata_dispatch* d, uint64_t offGate, uint64_t offUp
     float* const gu[2] = {g, u};
     const int Ng[2] = {F, F};
     if ((rc = prefill_f16_batch(d, 2, offs, names, gu, Ng, h, M, H, stream))) return rc;
-    for (int i = 0; i < 2; i++)
-        if (kata_dispatch_i8(d, names[i]) &&
-            (rc = kata_dispatch_prefill(d, offs[i], h, gu[i], M, H, F, names[i], A8, SX, M, stream)))
-            return rc;
+    bool quantised = false;                          // quantise h once for its int8 matrices
+    for (int i = 0; i < 2; i++) {
+        if (!kata_dispatch_i8(d, names[i])) continue;
+        if (!quantised && (rc = kata_quant_rows_i8(h, A8, SX, M, H, M, stream))) return rc;
+        quantised = true;
+        if ((rc = kata_gemm_ptq1_i8(A8, SX, M, d->wbase + offs[i], gu[i], KATA_F32, F, M, H, F, stream))) return rc;
+    }
     if ((rc = kata_rms_fwht(g, u, gs_down, t, KATA_F16, KATA_X_ROWS, F, M, 1, stream))) return rc;
     return kata_dispatch_prefill(d, offDown, t, out, M, F, H, "down", A8, SX, M, stream);
 }

@@ -32,7 +32,7 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "gemm_reg.h"
+#include "gemm_ptq1_copy.h"
 
 namespace kata {
 
@@ -40,77 +40,31 @@ namespace {
 
 using rg::u16x2;
 
-__host__ __device__ constexpr uint32_t p3x2(int n) {
-    return n == 0 ? 0x00010001u : n == 1 ? 0x00030003u : n == 2 ? 0x00090009u : n == 3 ? 0x001b001bu : 0x00510051u;
-}
-// the bytes (b0, b1) / (b2, b3) of w in 16-bit lanes (v_perm selector 0x0c is a zero byte)
-__device__ inline u16x2 bytes01(uint32_t w) { return __builtin_bit_cast(u16x2, __builtin_amdgcn_perm(0u, w, 0x0c010c00u)); }
-__device__ inline u16x2 bytes23(uint32_t w) { return __builtin_bit_cast(u16x2, __builtin_amdgcn_perm(0u, w, 0x0c030c02u)); }
-
 // PTQ1_0 weights as B operand registers.  Lane half lh of column c takes chunk 2 kk + lh (8
 // consecutive k) of every 16-k step kk of a block: for kk < 5 digit kk of qs bytes 8 lh .. 8 lh
 // + 7; for kk = 5, 6 digit 2 (kk - 5) + lh of bytes 16..23; for kk = 7 digit 4 of those (lh = 0)
 // or the qh bytes, digit j for pair j (lh = 1).
-struct Ptq1F16 {
+struct Ptq1F16 : Ptq1Copy {
     static constexpr bool TWO_FORMS = true;
-    static constexpr int kBlockB = kBlockBytes;   // bytes of 128 k of a row
-    static constexpr int GROUP = 2;               // blocks per copied group: 56 bytes of a row
-    template <class C>
-    static constexpr int copies() {
-        static_assert(C::BN * 4 % C::THREADS == 0, "whole weight copies per thread");
-        return C::BN * 4 / C::THREADS;
-    }
-    template <class C>
-    static constexpr int slot_bytes() { return C::BN * 64; }
 
-    const uint8_t* wbase[4];                      // copy sources: per instruction a uniform row base
-    uint32_t wvo[4];                              // and this lane's offset (full group)
-    uint32_t wsingle;                             // added to it in a group of one block
-    uint32_t w_lds;
-    uint32_t rd;                                  // LDS address of this lane's row (tile 0) in slot 0
     uint32_t o_own0, o_p1, o_own10, o_own11, o_p2, o_p3;
-    int lh, nblk;
+    int lh;
     uint32_t wn[2][5];                            // next block's words: own half, bytes 16..27
     u16x2 m[2][4];                                // remainders of the digits taken so far
     uint32_t w4[2], w5[2], w6[2];
     v2h dd[2], S[2];
 
-    // Copies: the 56 bytes of a row's group are four 16-byte pieces at 0, 16, 32, 40 (a last
-    // group of one block: 0, 12), so no copy reads past the row; row r's piece p sits in slot
-    // p ^ ((r >> 2) & 3) of its 64 LDS bytes.
     template <class C>
     __device__ inline void init(const uint8_t* W, int nbk, int kb0, int nb, int n0, int N, int tid, int wave, int wc,
                                 int l32, int lh_, uint32_t Ws) {
-        const uint32_t row_bytes = (uint32_t)nbk * kBlockBytes;
-        constexpr int RPI = C::THREADS / 4;
+        init_copy<C>(W, nbk, kb0, nb, n0, N, tid, wave, wc, l32, Ws);
         lh = lh_;
-        nblk = nb;
-#pragma unroll
-        for (int i = 0; i < copies<C>(); i++) {
-            const int r0 = min(n0 + i * RPI, N - 1), r = tid / 4;
-            const int p = (tid & 3) ^ (((i * RPI + r) >> 2) & 3);
-            wbase[i] = W + (size_t)r0 * row_bytes + (size_t)kb0 * kBlockBytes;
-            wvo[i] = (uint32_t)min(r, N - 1 - r0) * row_bytes + (p < 3 ? 16u * p : 40u);
-        }
-        const int p = (tid & 3) ^ ((tid >> 4) & 3);
-        wsingle = p == 0 ? 0u : (uint32_t)(12 - (p < 3 ? 16 * p : 40));
-        w_lds = Ws + 1024u * wave;
-        rd = Ws + (wc * 32 * C::NT + l32) * 64;
-        const uint32_t f = (uint32_t)(l32 >> 2) & 3u;
-        o_own0 = (f << 4) + 8u * lh;
-        o_p1 = (1u ^ f) << 4;
-        o_p2 = ((2u ^ f) << 4) + 12u;
-        o_p3 = ((3u ^ f) << 4) + 8u;
-        o_own10 = lh ? ((2u ^ f) << 4) + 4u : ((1u ^ f) << 4) + 12u;
-        o_own11 = ((2u ^ f) << 4) + (lh ? 8u : 0u);
-    }
-    template <class C>
-    __device__ inline void issue(int g, int slot, int i0, int i1) {
-        const uint32_t add = 2 * g + 1 == nblk ? wsingle : 0u;
-#pragma unroll
-        for (int i = i0; i < i1; i++)
-            rg::dma16(wbase[i] + (size_t)g * (2 * kBlockBytes), wvo[i] + add,
-                      w_lds + slot * slot_bytes<C>() + i * (C::THREADS * 16));
+        o_own0 = piece(0) + 8u * lh;
+        o_p1 = piece(1);
+        o_p2 = piece(2) + 12u;
+        o_p3 = piece(3) + 8u;
+        o_own10 = lh ? piece(2) + 4u : piece(1) + 12u;
+        o_own11 = piece(2) + (lh ? 8u : 0u);
     }
     template <class C, int J>
     __device__ inline void read(int g, int slot, int nb) {

@@ -17,6 +17,7 @@
 // four MFMAs, groups ascending.
 #include "common.h"
 #include "launch.h"
+#include "gemm_ptq1_copy.h"
 #include "gemm_tile.h"
 #include <utility>
 
@@ -65,11 +66,6 @@ __global__ __launch_bounds__(256) void k_quant_rows(const _Float16* __restrict__
     }
     *(uint2*)(Q + o) = make_uint2(q[0], q[1]);
     if (sub == 0) SX[(size_t)g * ldS + m] = scale;
-}
-
-// digit multipliers 3^n in both 16-bit lanes
-__host__ __device__ constexpr uint32_t p3x2(int n) {
-    return n == 0 ? 0x00010001u : n == 1 ? 0x00030003u : n == 2 ? 0x00090009u : n == 3 ? 0x001b001bu : 0x00510051u;
 }
 
 // int8 trits (digit - 1) of the 4 bytes of w, in byte order: bytes 0, 1 at the digit of
@@ -326,6 +322,281 @@ __global__ __launch_bounds__(64 * (kCW + 4)) void k_gemm_ptq1_i8(const int8_t* _
     }
 }
 
+// ---------------------------------------------------------------------------------------
+// Short tiles (32, 64 or 128 rows by 256 columns), on the skeleton of the fp16 GEMM
+// (gemm_reg.h): wave w owns all rows and columns 32w..32w+31, and each lane decodes the trits
+// of its own column straight into the MFMA's B registers.  A stage is one 128-group: its A
+// rows (128 bytes, the byte layout of an fp16 stage of 64 k), its row scales, and four
+// 32-k steps of v_mfma_i32_32x32x32_i8; the finished int32 tiles are folded into fp32 (groups
+// ascending, the tall kernel's expression) after the next group's first decode.  The tall kernel computes 256 rows whatever their
+// number: 28 / 41 / 100 rows of 5120 -> 17408 54.5 / 54.6 / 56.2 -> 25.4 / 29.8 / 40.0 us, of 17408 -> 5120
+// 42.0 / 42.5 / 43.4 -> 23.9 / 26.9 / 37.  From about 150 rows it is the faster one (200 rows 57.8
+// against 64): here every 128-row tile decodes its weights and folds 3 instructions per output
+// and group beside them (about 330 vector instructions per 16 MFMAs).
+namespace short_i8 {
+
+using rg::lds_ld;
+using rg::u16x2;
+using rg::u32x2;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+template <int MT_>
+struct Cfg {
+    static constexpr int MT = MT_, NT = 1, NWR = 1, NWC = 8, WAVES = 8, THREADS = 512;
+    static constexpr int BM = 32 * MT, BN = 256, DA = 2, DW = 2, ABUF = DA + 1;
+    static constexpr int ASTAGE = BM * 128;                      // A bytes of a stage
+    static constexpr int SXROWS = BM < 64 ? 64 : BM;             // row scales of a stage
+    static constexpr int NA = BM * 8 >= THREADS ? BM * 8 / THREADS : 1;
+    static constexpr int kSx = ABUF * ASTAGE, kW = kSx + ABUF * SXROWS * 4;
+    static constexpr int kLds = kW + (DW + 1) * BN * 64;
+};
+
+// B operand of 32-k step kk (16 consecutive k per lane: chunk 2 kk + lh of the block): digit 2 kk +
+// lh of qs bytes 0..15 for kk < 2; then digit 4 of those (lh = 0) or digits 0, 1 of bytes 16..23;
+// then digits 2, 3 of bytes 16..23 (lh = 0) or their digit 4 and the qh bytes.
+struct Trits : Ptq1Copy {
+    int lh;
+    uint32_t wn[7], w4, w5, w6;
+    u16x2 m[8];                                    // remainders of bytes 0..15
+    float d;
+
+    template <class C, int J>
+    __device__ inline void read(int g, int slot, int nb) {
+        const uint32_t p = rd + slot * slot_bytes<C>();
+        if constexpr (J == 0) {
+            const u32x4 a = lds_ld<u32x4>(p + piece(0));
+            const uint32_t q = p + piece(1) + (2 * g + 1 == nb ? 4u : 0u);
+#pragma unroll
+            for (int i = 0; i < 4; i++) wn[i] = a[i];
+#pragma unroll
+            for (int i = 0; i < 3; i++) wn[4 + i] = lds_ld<uint32_t>(q + 4 * i);
+        } else {
+            wn[0] = lds_ld<uint32_t>(p + piece(1) + 12);
+            const u32x4 a = lds_ld<u32x4>(p + piece(2));
+            const u32x2 b = lds_ld<u32x2>(p + piece(3) + 8);
+#pragma unroll
+            for (int i = 0; i < 4; i++) wn[1 + i] = a[i];
+            wn[5] = b[0];
+            wn[6] = b[1];
+        }
+    }
+    // unpack the block read ahead; its scale
+    __device__ inline float begin() {
+        const u16x2 mul = __builtin_bit_cast(u16x2, lh ? p3x2(1) : p3x2(0));
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            m[2 * i] = (bytes01(wn[i]) * mul) & (u16x2){0xff, 0xff};
+            m[2 * i + 1] = (bytes23(wn[i]) * mul) & (u16x2){0xff, 0xff};
+        }
+        w4 = wn[4];
+        w5 = wn[5];
+        w6 = wn[6];
+        return half_bits_to_float(w6 >> 16);
+    }
+    template <int kk>
+    __device__ inline v4i chunk() {
+        const u16x2 lo8 = {0xff, 0xff}, nine = {9, 9};
+        u16x2 r[8];                                // the digits' remainders, four bytes per dword pair
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const uint32_t w = j & 2 ? w5 : w4;
+            const u16x2 n = j & 1 ? bytes23(w) : bytes01(w);
+            auto pick = [&](u16x2 a, u16x2 b) {    // a for lh = 0, b for lh = 1
+                return __builtin_bit_cast(u16x2, lh ? __builtin_bit_cast(uint32_t, b) : __builtin_bit_cast(uint32_t, a));
+            };
+            auto mulc = [&](int a, int b) { return __builtin_bit_cast(u16x2, lh ? p3x2(b) : p3x2(a)); };
+            if constexpr (kk < 2) {
+                if constexpr (kk == 1) m[j] = (m[j] * nine) & lo8;
+                r[j] = m[j];
+            } else if constexpr (kk == 2) {
+                r[j] = (pick(m[j], n) * mulc(2, j < 4 ? 0 : 1)) & lo8;
+            } else {
+                r[j] = j < 4 ? (n * mulc(2, 4)) & lo8 : (pick(n, bytes01(w6)) * mulc(3, j - 4)) & lo8;
+            }
+        }
+        v4i o;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            // 3 m - 256 has the trit (digit - 1) in its high byte
+            const u16x2 a = r[2 * i] * (u16x2){3, 3} + (u16x2){0xff00, 0xff00};
+            const u16x2 b = r[2 * i + 1] * (u16x2){3, 3} + (u16x2){0xff00, 0xff00};
+            o[i] = (int)__builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), 0x07050301u);
+        }
+        return o;
+    }
+};
+
+template <class C, bool C_F16>
+__global__ __launch_bounds__(512, 2) void k_gemm_i8_short(const int8_t* __restrict__ A8, const float* __restrict__ SX,
+                                                          int ldS, rg::Mats P, float* __restrict__ ws, int M, int K,
+                                                          GemmJobs J) {
+    constexpr int MT = C::MT, DA = C::DA, DW = C::DW, NA = C::NA, ABUF = C::ABUF, SPG = 2;
+    constexpr int NW = Ptq1Copy::copies<C>();
+    static_assert((DW - 1) * SPG >= DA, "a group's copies, spread over two stages, land in time");
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, lh = lane >> 5;
+    const int nbk = K >> 7;
+    int job, tile, kb0, nb;
+    gemm_job(J, nbk, job, tile, kb0, nb);
+    const int m0 = (tile / J.G) * C::BM, mi = rg::mat_of(P, tile % J.G), n0 = (tile % J.G - P.g0[mi]) * C::BN;
+    const int N = P.N[mi];
+    const int ng = (nb + 1) / 2;
+
+    // A copies: instruction i copies rows 64 i .. + 63 of a stage (32-row tiles: the upper waves
+    // repeat the lower ones'), chunk c of row r at c ^ ((r >> 1) & 7); limited to row M - 1
+    const int arow = (tid >> 3) & (C::BM < 64 ? 31 : 63);
+    const uint32_t avo = (uint32_t)arow * (uint32_t)K + (uint32_t)(((tid & 7) ^ ((arow >> 1) & 7)) << 4);
+    const uint32_t a_lds = 1024u * (C::BM < 64 ? wave & 3 : wave);
+    auto issue_a = [&](int st) {
+        const int buf = st % ABUF;
+        const int8_t* ko = A8 + (size_t)(kb0 + min(st, nb - 1)) * 128;
+#pragma unroll
+        for (int i = 0; i < NA; i++) {
+            const int r0 = min(m0 + i * 64, M - 1);
+            const uint32_t lim = M - 1 - r0 < 64 ? (uint32_t)(M - 1 - r0) * (uint32_t)K + 112u : 0xffffffffu;
+            rg::dma16(ko + (size_t)r0 * K, min(avo, lim), a_lds + buf * C::ASTAGE + i * 8192);
+        }
+        // the stage's row scales, one dword per lane: wave w rows 64 (w % (SXROWS / 64)) + lane
+        const int rg64 = wave & (C::SXROWS / 64 - 1);
+        rg::dma4(SX + (size_t)(kb0 + min(st, nb - 1)) * ldS, 4u * (uint32_t)min(m0 + 64 * rg64 + lane, M - 1),
+                 C::kSx + buf * (C::SXROWS * 4) + 256u * rg64);
+    };
+    Trits dec;
+    dec.lh = lh;
+    dec.template init_copy<C>(P.W[mi], nbk, kb0, nb, n0, N, tid, wave, wave, l32, C::kW);
+    auto issue_w = [&](int g, int i0, int i1) { dec.template issue<C>(min(g, ng - 1), g % (DW + 1), i0, i1); };
+
+    v16f acc[MT];
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int q = 0; q < 16; q++) acc[i][q] = 0.0f;
+    // copies that may fly when stage sp is awaited: the DA - 1 stages after it and the weight parts
+    // issued with them
+    auto vm_of = [](int sp) constexpr {
+        int n = (DA - 1) * (NA + 1);
+        for (int j = sp - DA + 1; j < sp; j++) n += ((j + SPG) % SPG + 1) * NW / SPG - (j + SPG) % SPG * NW / SPG;
+        return n;
+    };
+    rg::unroll<DW * SPG>([&](auto ic) {
+        constexpr int j = decltype(ic)::value - DW * SPG, sp = (j + DW * SPG) % SPG;
+        issue_w((j - sp) / SPG + DW, sp * NW / SPG, (sp + 1) * NW / SPG);
+        if constexpr (j >= -DA) issue_a(j + DA);
+    });
+    const uint32_t a_row = (uint32_t)l32 * 128u + (uint32_t)((lh ^ ((l32 >> 1) & 7)) << 4);
+    const uint32_t sx_row = C::kSx + 4u * (8 * ((lane & 15) >> 2) + 4 * lh + (lane & 3));
+    v4i af[2][MT], bf[2];
+    auto frags = [&](int kk, int buf, v4i (&f)[MT]) {
+        const uint32_t at = buf * C::ASTAGE + (a_row ^ (uint32_t)(kk << 5));
+#pragma unroll
+        for (int i = 0; i < MT; i++) f[i] = lds_ld<v4i>(at + i * 4096);
+    };
+    rg::wait_vm<vm_of(0)>();
+    rg::barrier_lds();
+    dec.template read<C, 0>(0, 0, nb);
+    frags(0, 0, af[0]);
+    float d = dec.begin();
+    bf[0] = dec.template chunk<0>();
+    int s = 0, abuf = 0;
+    v16i I[MT];
+    float sx[MT];
+    static_assert(NW == 2 && vm_of(0) == vm_of(1), "one weight copy per stage: every stage waits alike");
+    for (int b = 0; b < nb; b++) {
+        const int g = b >> 1;
+        if (b & 1) dec.template read<C, 0>(g + 1, (g + 1) % (DW + 1), nb);      // the next block's words
+        else dec.template read<C, 1>(g, g % (DW + 1), nb);
+        rg::unroll<4>([&](auto kc) {
+            constexpr int kk = decltype(kc)::value, cur = kk & 1, nxt = cur ^ 1;
+            if constexpr (kk == 3) {                 // the next stage has landed, this one's fragments are held
+                ++s;
+                abuf = abuf + 1 == ABUF ? 0 : abuf + 1;
+                rg::wait_vm<vm_of(0)>();
+                rg::barrier_lds();
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            frags((kk + 1) % 4, abuf, af[nxt]);
+            if constexpr (kk == 0) {
+#pragma unroll
+                for (int i = 0; i < MT; i++) sx[i] = lds_ld<float>(sx_row + abuf * (C::SXROWS * 4) + i * 128);
+            }
+#pragma unroll
+            for (int i = 0; i < MT; i++) {
+                if constexpr (kk == 0) {
+#pragma unroll
+                    for (int q = 0; q < 16; q++) I[i][q] = 0;
+                }
+                I[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[cur][i], bf[cur], I[i], 0, 0, 0);
+            }
+            const float dg = d;
+            if constexpr (kk == 3) d = dec.begin();
+            bf[nxt] = dec.template chunk<(kk + 1) % 4>();
+            if constexpr (kk == 3) {
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < MT; i++) fold_tile(acc[i], I[i], dg, sx[i], std::make_integer_sequence<int, 16>());
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (kk == 0) {
+                if (b & 1) issue_w(g + DW, 1, 2);
+                else issue_w(g + DW, 0, 1);
+            }
+            if constexpr (kk == 1) issue_a(s + DA);
+        });
+    }
+    rg::wait_vm<0>();
+
+    const int gc = wave * 32 + l32;                  // tile column
+    if (job >= J.n_full) {
+        float* T = ws + (size_t)(job - J.n_full) * (C::BM * C::BN);
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int q = 0; q < 16; q++) {
+                const int r = i * 32 + 8 * (q >> 2) + 4 * lh + (q & 3);
+                if (m0 + r < M) T[r * C::BN + gc] = acc[i][q];
+            }
+        return;
+    }
+    void* Cp = P.C[mi];
+    const int ldc = P.ldc[mi], gn = n0 + gc;
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int q = 0; q < 16; q++) {
+            const int gm = m0 + i * 32 + 8 * (q >> 2) + 4 * lh + (q & 3);
+            if (gm < M && gn < N) {
+                if (C_F16) ((_Float16*)Cp)[(size_t)gm * ldc + gn] = (_Float16)acc[i][q];
+                else ((float*)Cp)[(size_t)gm * ldc + gn] = acc[i][q];
+            }
+        }
+}
+
+// us per 128-group of a tile (see rg::Shape), fitted to 28..2500 rows of three model shapes
+constexpr rg::Shape kShapes[3] = {{32, 256, 1.1f, 1.1f, 2}, {64, 256, 1.3f, 1.3f, 2}, {128, 256, 1.75f, 1.8f, 2}};
+
+template <class C>
+hipError_t launch_cfg(const int8_t* A8, const float* SX, int ldS, const rg::Mats& P, float* ws, int c_dtype, bool v4, int M,
+                      int K, const GemmJobs& J, hipStream_t s) {
+    static_assert(C::kLds <= 160 * 1024, "LDS");
+    static const hipError_t attr = [] {
+        hipError_t e = hipFuncSetAttribute((const void*)k_gemm_i8_short<C, true>, hipFuncAttributeMaxDynamicSharedMemorySize, C::kLds);
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute((const void*)k_gemm_i8_short<C, false>, hipFuncAttributeMaxDynamicSharedMemorySize, C::kLds);
+        return e;
+    }();
+    if (attr != hipSuccess) return attr;
+    if (c_dtype == 1)
+        hipLaunchKernelGGL((k_gemm_i8_short<C, true>), dim3(J.n_jobs), dim3(512), C::kLds, s, A8, SX, ldS, P, ws, M, K, J);
+    else
+        hipLaunchKernelGGL((k_gemm_i8_short<C, false>), dim3(J.n_jobs), dim3(512), C::kLds, s, A8, SX, ldS, P, ws, M, K, J);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    return rg::launch_pieces_sum<C::BM, C::BN>(ws, P, c_dtype, v4, M, J, s);
+}
+
+}  // namespace short_i8
+
 }  // namespace
 
 hipError_t launch_quant_rows(const uint16_t* X, int8_t* Q, float* SX, int M, int K, int ldS, hipStream_t s) {
@@ -350,7 +621,48 @@ hipError_t launch_gemm_i8(const int8_t* A8, const float* SX, int ldS, const uint
     float* ws = nullptr;
     hipError_t e = gemm_device(false, s, &n_cu, &ws);
     if (e != hipSuccess) return e;
-    const GemmJobs J = plan_gemm_jobs(M, N, K, BM, BN, n_cu);   // one workgroup per CU
+    // The short tiles where the cost model has them cheaper than the tall kernel's schedule (whole
+    // rounds of 256 x 128 tiles at 1.3 us per group, the rest in K pieces); their row offsets
+    // are 32-bit.
+    GemmJobs J = plan_gemm_jobs(M, N, K, BM, BN, n_cu);   // one workgroup per CU
+    if (K <= (1 << 23)) {
+        const int nbk = K / kGroup, G = (N + 255) / 256, rem = J.n_jobs - J.n_full;
+        auto rounds = [&](int jobs) { return (jobs + n_cu - 1) / n_cu; };
+        double tall = rounds(J.n_full) * (3.0 + nbk * 1.3);
+        if (rem) tall += 3.0 + (nbk + J.S - 1) / J.S * 1.3 + 4.0 + (double)rem * BM * BN * 8.0 / 4e6;
+        int k = -1;
+        auto choose = [&](bool pieces) {
+            rg::Plan best{};
+            for (int i = 0; i < 3; i++) {
+                const rg::Plan p = rg::plan(short_i8::kShapes[i], M, G, nbk, n_cu, pieces);
+                if (k < 0 || p.us < best.us) {
+                    best = p;
+                    k = i;
+                }
+            }
+            return best;
+        };
+        rg::Plan p = choose(true);
+        if (p.us < tall) {
+            if (p.J.n_jobs > p.J.n_full && gemm_device(true, s, &n_cu, &ws) != hipSuccess) {
+                (void)hipGetLastError();
+                k = -1;
+                p = choose(false);
+            }
+            rg::Mats P{};
+            P.W[0] = W;
+            P.C[0] = C;
+            P.N[0] = N;
+            P.ldc[0] = ldc;
+            for (int i = 1; i <= rg::kMaxMats; i++) P.g0[i] = 0x7fffffff;
+            const bool v4 = N % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)C & 15) == 0;
+            switch (k) {
+                case 0: return short_i8::launch_cfg<short_i8::Cfg<1>>(A8, SX, ldS, P, ws, c_dtype, v4, M, K, p.J, s);
+                case 1: return short_i8::launch_cfg<short_i8::Cfg<2>>(A8, SX, ldS, P, ws, c_dtype, v4, M, K, p.J, s);
+                default: return short_i8::launch_cfg<short_i8::Cfg<4>>(A8, SX, ldS, P, ws, c_dtype, v4, M, K, p.J, s);
+            }
+        }
+    }
     if (J.n_jobs > J.n_full && (e = gemm_device(true, s, &n_cu, &ws)) != hipSuccess) return e;
     if (c_dtype == 1)
         hipLaunchKernelGGL(k_gemm_ptq1_i8<true>, dim3(J.n_jobs), dim3(64 * (kCW + 4)), kLdsBytes, s, A8, SX, ldS, W, C, ldc, ws,

@@ -16,7 +16,6 @@
 #pragma once
 #include <algorithm>
 #include <array>
-#include <cstdlib>
 #include <utility>
 
 #include "common.h"
@@ -73,6 +72,14 @@ __device__ inline void unroll(F&& f) {
 __device__ inline void dma16(const void* base, uint32_t voff, uint32_t lds) {
     uint32_t saved;
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+                 : "=&s"(saved)
+                 : "v"(voff), "s"(base), "s"(lds)
+                 : "memory");
+}
+// the same, one dword per lane to lds + 4*lane
+__device__ inline void dma4(const void* base, uint32_t voff, uint32_t lds) {
+    uint32_t saved;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\tglobal_load_lds_dword %1, %2\n\ts_mov_b32 m0, %0"
                  : "=&s"(saved)
                  : "v"(voff), "s"(base), "s"(lds)
                  : "memory");
@@ -485,12 +492,6 @@ hipError_t launch(const Shape (&shapes)[sizeof...(Cs)], const _Float16* A, int l
         return best.J;
     };
     GemmJobs J = choose(true);
-#ifdef TUNE
-    if (const char* q = getenv("KBM")) {
-        k = atoi(q); J = plan(shapes[k], M, G, K / 128, n_cu, true).J;
-        if (const char* q2 = getenv("KS")) { const int T = (M + shapes[k].bm - 1) / shapes[k].bm * G, S = atoi(q2); if (S > K / 128 || S > 16 || (double)T * S * shapes[k].bm * shapes[k].bn > (double)n_cu * kPieceFloats) return hipErrorInvalidValue; J = S > 1 ? GemmJobs{G, 0, S, T * S} : GemmJobs{G, T, 1, T}; }
-    }
-#endif
     if (J.n_jobs > J.n_full && gemm_device(true, s, &n_cu, &ws) != hipSuccess) {
         // no workspace (the stream's first call is captured, or memory is short): whole tiles
         (void)hipGetLastError();

@@ -21,7 +21,9 @@ def _weights(dev, K, N, seed, big):
     rng = np.random.default_rng(seed)
     t = rng.integers(-1, 2, (N, K)).astype(np.int8)
     d = np.abs(rng.normal(0, 0.02, (N, K // 128)))
-    if big:                                     # blocks at and above 1, tiny and zero scales
+    if big == "tiny":                           # subnormal fp16 scales, in the fast decode form
+        d *= 2e-5
+    elif big:                                   # blocks at and above 1, tiny and zero scales
         d[:, ::3] *= 5000.0
         d[1::7] = 1.0
         d[::5, 1::4] = 3e-7
@@ -35,7 +37,7 @@ def _check(C, A, W, K, N):
     assert err < 1e-5, err
 
 
-@pytest.mark.parametrize("big", [False, True])
+@pytest.mark.parametrize("big", [False, "tiny", True])
 @pytest.mark.parametrize("M", [1, 31, 32, 33, 64, 65, 127, 129, 256, 257, 700])
 @pytest.mark.parametrize("K,N", [(128, 257), (384, 1000), (2176, 256), (5120, 255)])
 def test_tile_edges(dev, M, K, N, big):
