@@ -24,6 +24,8 @@
 #include "gemv_operand.h"
 #include "launch.h"
 
+#include <type_traits>
+
 namespace kata {
 
 namespace {
@@ -31,71 +33,124 @@ namespace {
 constexpr float kRmsEps = 1e-6f;   // config/kata_m6.h:21
 __constant__ DenseImgOff kOperandOff = make_dense_img_off();
 
-__device__ inline float wave_sum(float a) {
+// The value of lane l ^ m for m = 1, 2 (DPP quad permutations), 4 (DPP row shifts: the partner is
+// in the lane's row of 16, l + m when bit m is clear, l - m when set; bound_ctrl reads 0 for
+// sources outside the row, so the unselected shift is harmless) and 8 (DPP row rotation).  Both
+// shifts are computed in every lane before the select: a conditional expression with the DPP
+// moves as operands evaluates one per lane, which becomes a branch in which the moves read
+// disabled source lanes (zeros).
+template <int m>
+__device__ inline float partner(float v, int lane) {
+    const int iv = __builtin_bit_cast(int, v);
+    int pv;
+    if constexpr (m == 1) {
+        pv = __builtin_amdgcn_mov_dpp(iv, 0xB1, 0xf, 0xf, true);           // quad_perm [1, 0, 3, 2]
+    } else if constexpr (m == 2) {
+        pv = __builtin_amdgcn_mov_dpp(iv, 0x4E, 0xf, 0xf, true);           // quad_perm [2, 3, 0, 1]
+    } else if constexpr (m == 4) {
+        const int up = __builtin_amdgcn_mov_dpp(iv, 0x104, 0xf, 0xf, true);   // row_shl:4
+        const int dn = __builtin_amdgcn_mov_dpp(iv, 0x114, 0xf, 0xf, true);   // row_shr:4
+        pv = lane & 4 ? dn : up;
+    } else {
+        static_assert(m == 8, "partner in the row");
+        pv = __builtin_amdgcn_mov_dpp(iv, 0x128, 0xf, 0xf, true);          // row_ror:8
+    }
+    return __builtin_bit_cast(float, pv);
+}
+// For m = 16, 32: lo = the value of the lane with bit m clear, hi = of the one with it set (both
+// in both lanes; a vector instruction, where a cross-lane permute goes through LDS)
+template <int m>
+__device__ inline void halves(float v, float& lo, float& hi) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    if constexpr (m == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        lo = __builtin_bit_cast(float, (uint32_t)r[0]);
+        hi = __builtin_bit_cast(float, (uint32_t)r[1]);
+    } else {
+        const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        lo = __builtin_bit_cast(float, (uint32_t)r[0]);
+        hi = __builtin_bit_cast(float, (uint32_t)r[1]);
+    }
+}
+
+__device__ inline float wave_sum(float a, int lane) {
     // fixed-order butterfly over the 64 lanes
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o);
+    float lo, hi;
+    halves<32>(a, lo, hi);
+    a = lo + hi;
+    halves<16>(a, lo, hi);
+    a = lo + hi;
+    a += partner<8>(a, lane);
+    a += partner<4>(a, lane);
+    a += partner<2>(a, lane);
+    a += partner<1>(a, lane);
     return a;
 }
 
-// natural-order butterflies: for bit h the pair (k, k | h) becomes (a + b, a - b)
-__device__ inline void fwht1024(float (&v)[4], int tid, float* xs) {
+// natural-order butterflies over NB blocks of 1024: for bit h the pair (k, k | h) becomes
+// (a + b, a - b).  The blocks go through each level together: two barriers for all of them, and
+// the cross-lane moves of one block fill the waits of another's.
+template <int NB>
+__device__ inline void fwht1024(float (&v)[NB][4], int tid, float* xs) {
+#pragma clang fp contract(off)                   // the sums of rounded products, in every caller
     const int lane = tid & 63;
-    float a = v[0] + v[1], b = v[0] - v[1], c = v[2] + v[3], d = v[2] - v[3];
-    v[0] = a + c;
-    v[1] = b + d;
-    v[2] = a - c;
-    v[3] = b - d;
-    // the partner lane l ^ m: m = 1, 2 by DPP quad permutations, m = 4, 8 by DPP row shifts
-    // (the partner is in the lane's row of 16: l + m when bit m is clear, l - m when set;
-    // bound_ctrl reads 0 for sources outside the row, so the unselected shift is harmless),
-    // m = 16, 32 by a cross-lane permute.  Both shifts are computed in every lane before the
-    // select: a conditional expression with the DPP moves as operands evaluates one per lane,
-    // which becomes a branch in which the moves read disabled source lanes (zeros).
 #pragma unroll
-    for (int k = 0; k < 6; k++) {
-        const int m = 1 << k;
+    for (int n = 0; n < NB; n++) {
+        const float a = v[n][0] + v[n][1], b = v[n][0] - v[n][1], c = v[n][2] + v[n][3], d = v[n][2] - v[n][3];
+        v[n][0] = a + c;
+        v[n][1] = b + d;
+        v[n][2] = a - c;
+        v[n][3] = b - d;
+    }
+    // the pair (l, l ^ m): the lane with bit m clear takes the sum, the other the difference
+    auto level = [&](auto mc) {
+        constexpr int m = decltype(mc)::value;
         const bool hi = lane & m;
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int iv = __builtin_bit_cast(int, v[r]);
-            int pv;
-            if (k == 0) {
-                pv = __builtin_amdgcn_mov_dpp(iv, 0xB1, 0xf, 0xf, true);   // quad_perm [1, 0, 3, 2]
-            } else if (k == 1) {
-                pv = __builtin_amdgcn_mov_dpp(iv, 0x4E, 0xf, 0xf, true);   // quad_perm [2, 3, 0, 1]
-            } else if (k == 2) {
-                const int up = __builtin_amdgcn_mov_dpp(iv, 0x104, 0xf, 0xf, true);   // row_shl:4
-                const int dn = __builtin_amdgcn_mov_dpp(iv, 0x114, 0xf, 0xf, true);   // row_shr:4
-                pv = hi ? dn : up;
-            } else if (k == 3) {
-                const int up = __builtin_amdgcn_mov_dpp(iv, 0x108, 0xf, 0xf, true);   // row_shl:8
-                const int dn = __builtin_amdgcn_mov_dpp(iv, 0x118, 0xf, 0xf, true);   // row_shr:8
-                pv = hi ? dn : up;
-            } else {
-                pv = __shfl_xor(iv, m);
+        for (int n = 0; n < NB; n++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                float& x = v[n][r];
+                if constexpr (m <= 8) {
+                    const float p = partner<m>(x, lane);
+                    x = hi ? p - x : x + p;
+                } else {
+                    float l, h;
+                    halves<m>(x, l, h);
+                    x = l + (hi ? -h : h);
+                }
             }
-            const float p = __builtin_bit_cast(float, pv);
-            v[r] = hi ? p - v[r] : v[r] + p;
-        }
-    }
+    };
+    level(std::integral_constant<int, 1>{});
+    level(std::integral_constant<int, 2>{});
+    level(std::integral_constant<int, 4>{});
+    level(std::integral_constant<int, 8>{});
+    level(std::integral_constant<int, 16>{});
+    level(std::integral_constant<int, 32>{});
     // bits 8-9: element k = 4 tid + r; thread t then owns elements t + 256 j (j = 0..3)
 #pragma unroll
-    for (int r = 0; r < 4; r++) xs[4 * tid + r] = v[r];
-    __syncthreads();
-    float e[4];
+    for (int n = 0; n < NB; n++)
 #pragma unroll
-    for (int j = 0; j < 4; j++) e[j] = xs[tid + 256 * j];
-    const float a2 = e[0] + e[1], b2 = e[0] - e[1], c2 = e[2] + e[3], d2 = e[2] - e[3];
-    e[0] = a2 + c2;
-    e[1] = b2 + d2;
-    e[2] = a2 - c2;
-    e[3] = b2 - d2;
-#pragma unroll
-    for (int j = 0; j < 4; j++) xs[tid + 256 * j] = e[j];
+        for (int r = 0; r < 4; r++) xs[1024 * n + 4 * tid + r] = v[n][r];
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < 4; r++) v[r] = xs[4 * tid + r] * 0.03125f;
+    for (int n = 0; n < NB; n++) {
+        float e[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) e[j] = xs[1024 * n + tid + 256 * j];
+        const float a2 = e[0] + e[1], b2 = e[0] - e[1], c2 = e[2] + e[3], d2 = e[2] - e[3];
+        e[0] = a2 + c2;
+        e[1] = b2 + d2;
+        e[2] = a2 - c2;
+        e[3] = b2 - d2;
+#pragma unroll
+        for (int j = 0; j < 4; j++) xs[1024 * n + tid + 256 * j] = e[j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < NB; n++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) v[n][r] = xs[1024 * n + 4 * tid + r] * 0.03125f;
 }
 
 __device__ inline float silu(float x) { return x / (1.0f + expf(-x)); }
@@ -188,70 +243,92 @@ __device__ inline void store_operand_wide(const float (&v)[4], uint2 offw, int t
     }
 }
 
-template <int NB>
+template <int NB, bool NORM>
 __global__ __launch_bounds__(256) void k_norm_fwht(const float* __restrict__ src, const float* __restrict__ src2,
                                                    const float* __restrict__ gs, void* __restrict__ out, int out_dtype,
                                                    int out_layout, float* __restrict__ xnew,
                                                    const float* __restrict__ gamma, void* __restrict__ hout,
                                                    int flags, int W, int mode) {
-    __shared__ float xs[1024];
+    __shared__ float xs[NB * 1024];
     __shared__ float part[4];
     const int tid = threadIdx.x;
-    const int m = NB == 1 ? blockIdx.y : blockIdx.x, blk0 = NB == 1 ? blockIdx.x : 0;
+    const int m = blockIdx.x, blk0 = blockIdx.y;          // rows in x: y ends at 65535
     const size_t ro = (size_t)m * W;
     // the operand form's image offsets of this thread's 4 elements, loaded first (their
     // latency then overlaps the row loads)
     uint2 offw = make_uint2(0, 0);
     if (out_dtype == 2) {
-        const int M = NB == 1 ? gridDim.y : gridDim.x;
+        const int M = gridDim.x;
         offw = *(const uint2*)&kOperandOff.v[M <= 2 ? M - 1 : 2][(4 * tid) & 127];
     }
+    // Few rows are bound by latency: every load of the blocks and of the row's sum of squares is
+    // issued before the first is used, from addresses that are always valid instead of under
+    // branches, whose joins wait.  x + y, norm and operand at W = 5120 in a graph: 4.14 -> 3.40 us
+    // at 1 row, 4.39 -> 3.68 at 6 (2.1 us of it are the launch).
+    float4 g[NB], gm[NORM ? NB : 1];
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        const int base = (blk0 + b) * 1024 + 4 * tid;
+        g[b] = *(const float4*)(gs + base);
+        if constexpr (NORM) gm[b] = *(const float4*)((flags & 4 ? gamma : gs) + base);
+    }
     // v = x (+ y) of this thread's elements 1024 (blk0 + b) + 4 tid + r, b < NB
-    float s[NB][4];
-    if (mode == 0) {
+    [[maybe_unused]] float s[NORM ? NB : 1][4];
+    float inv = 1.0f;
+    if constexpr (NORM) {
+        constexpr int NR = 6;                    // 1024-blocks of the row in flight
+        const float* const yrow = (flags & 1 ? src2 : src) + ro;
+        float4 ra[NB == 1 ? NR : 1], rc[NB == 1 ? NR : 1];
+        if constexpr (NB == 1) {
+#pragma unroll
+            for (int j = 0; j < NR; j++) {
+                const int i = 4 * tid + (1024 * j < W ? 1024 * j : 0);
+                ra[j] = *(const float4*)(src + ro + i);
+                rc[j] = *(const float4*)(yrow + i);
+            }
+        }
 #pragma unroll
         for (int b = 0; b < NB; b++) {
             const int base = (blk0 + b) * 1024 + 4 * tid;
             const float4 a = *(const float4*)(src + ro + base);
-            float4 c = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (flags & 1) c = *(const float4*)(src2 + ro + base);
+            float4 c = *(const float4*)(yrow + base);
+            if (!(flags & 1)) c = make_float4(0.f, 0.f, 0.f, 0.f);
             s[b][0] = a.x + c.x;
             s[b][1] = a.y + c.y;
             s[b][2] = a.z + c.z;
             s[b][3] = a.w + c.w;
         }
-    }
-    float inv = 1.0f;
-    if (mode == 0) {
         float ss = 0.0f;
-        if (NB == 1) {
-            for (int i = 4 * tid; i < W; i += 1024) {
-                const float4 a = *(const float4*)(src + ro + i);
-                float4 c = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (flags & 1) c = *(const float4*)(src2 + ro + i);
-                const float v0 = a.x + c.x, v1 = a.y + c.y, v2 = a.z + c.z, v3 = a.w + c.w;
-                ss += (v0 * v0 + v1 * v1) + (v2 * v2 + v3 * v3);
+        auto add = [&](const float4& a, float4 c) {
+            if (!(flags & 1)) c = make_float4(0.f, 0.f, 0.f, 0.f);
+            const float v0 = a.x + c.x, v1 = a.y + c.y, v2 = a.z + c.z, v3 = a.w + c.w;
+            ss += (v0 * v0 + v1 * v1) + (v2 * v2 + v3 * v3);
+        };
+        if constexpr (NB == 1) {
+#pragma unroll
+            for (int j = 0; j < NR; j++)
+                if (1024 * j < W) add(ra[j], rc[j]);
+            for (int i = 4 * tid + 1024 * NR; i < W; i += 1024) {
+                add(*(const float4*)(src + ro + i), *(const float4*)(yrow + i));
             }
         } else {
 #pragma unroll
             for (int b = 0; b < NB; b++) ss += (s[b][0] * s[b][0] + s[b][1] * s[b][1]) + (s[b][2] * s[b][2] + s[b][3] * s[b][3]);
         }
-        ss = wave_sum(ss);
+        ss = wave_sum(ss, tid & 63);
         if ((tid & 63) == 0) part[tid >> 6] = ss;
         __syncthreads();
         inv = 1.0f / sqrtf((part[0] + part[1] + part[2] + part[3]) / (float)W + kRmsEps);
     }
+    float v[NB][4];
 #pragma unroll
     for (int b = 0; b < NB; b++) {
         const int base = (blk0 + b) * 1024 + 4 * tid;
-        float v[4];
-        const float4 g = *(const float4*)(gs + base);
-        const float gv[4] = {g.x, g.y, g.z, g.w};
-        if (mode == 0) {
+        const float gv[4] = {g[b].x, g[b].y, g[b].z, g[b].w};
+        if constexpr (NORM) {
             if (flags & 2) *(float4*)(xnew + ro + base) = make_float4(s[b][0], s[b][1], s[b][2], s[b][3]);
             if (flags & 4) {
-                const float4 gm = *(const float4*)(gamma + base);
-                const float h[4] = {s[b][0] * inv * gm.x, s[b][1] * inv * gm.y, s[b][2] * inv * gm.z, s[b][3] * inv * gm.w};
+                const float h[4] = {s[b][0] * inv * gm[b].x, s[b][1] * inv * gm[b].y, s[b][2] * inv * gm[b].z, s[b][3] * inv * gm[b].w};
                 if (flags & 8) {
                     typedef _Float16 h4 __attribute__((ext_vector_type(4)));
                     *(h4*)((_Float16*)hout + ro + base) = h4{(_Float16)h[0], (_Float16)h[1], (_Float16)h[2], (_Float16)h[3]};
@@ -260,40 +337,45 @@ __global__ __launch_bounds__(256) void k_norm_fwht(const float* __restrict__ src
                 }
             }
 #pragma unroll
-            for (int r = 0; r < 4; r++) v[r] = s[b][r] * inv * gv[r];
+            for (int r = 0; r < 4; r++) v[b][r] = s[b][r] * inv * gv[r];
         } else if (mode == 1) {
             const float4 a = *(const float4*)(src + ro + base);
             const float4 c = *(const float4*)(src2 + ro + base);
             const float av[4] = {a.x, a.y, a.z, a.w}, cv[4] = {c.x, c.y, c.z, c.w};
 #pragma unroll
-            for (int r = 0; r < 4; r++) v[r] = silu(av[r]) * cv[r] * gv[r];
+            for (int r = 0; r < 4; r++) v[b][r] = silu(av[r]) * cv[r] * gv[r];
         } else if (mode == 2) {
+            const float4 a = *(const float4*)(src + ro + gdn_perm(base));    // base..base + 3 in one head
+            const float av[4] = {a.x, a.y, a.z, a.w};
 #pragma unroll
-            for (int r = 0; r < 4; r++) v[r] = src[ro + gdn_perm(base + r)] * gv[r];
+            for (int r = 0; r < 4; r++) v[b][r] = av[r] * gv[r];
         } else {
             const float4 a = *(const float4*)(src + ro + base);
             const float av[4] = {a.x, a.y, a.z, a.w};
 #pragma unroll
-            for (int r = 0; r < 4; r++) v[r] = av[r] * gv[r];
+            for (int r = 0; r < 4; r++) v[b][r] = av[r] * gv[r];
         }
-        fwht1024(v, tid, xs);
+    }
+    fwht1024(v, tid, xs);
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        const int base = (blk0 + b) * 1024 + 4 * tid;
         if (out_dtype == 2) {
-            const int M = NB == 1 ? gridDim.y : gridDim.x;
+            const int M = gridDim.x;
             if (M <= 2)
-                store_operand(v, offw, tid, blk0 + b, m, M, W, (uint8_t*)xs, (uint8_t*)out);
+                store_operand(v[b], offw, tid, blk0 + b, m, M, W, (uint8_t*)xs, (uint8_t*)out);
             else
-                store_operand_wide(v, offw, tid, blk0 + b, m, M, W, (uint8_t*)xs, (uint8_t*)out);
+                store_operand_wide(v[b], offw, tid, blk0 + b, m, M, W, (uint8_t*)xs, (uint8_t*)out);
         } else if (out_dtype == 0) {
-            *(float4*)((float*)out + ro + base) = make_float4(v[0], v[1], v[2], v[3]);
+            *(float4*)((float*)out + ro + base) = make_float4(v[b][0], v[b][1], v[b][2], v[b][3]);
         } else if (out_layout == 0) {
             typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-            *(h4*)((_Float16*)out + ro + base) = h4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+            *(h4*)((_Float16*)out + ro + base) = h4{(_Float16)v[b][0], (_Float16)v[b][1], (_Float16)v[b][2], (_Float16)v[b][3]};
         } else {
             _Float16* o = (_Float16*)out;        // [W][2]: token m at 2 i + m
 #pragma unroll
-            for (int r = 0; r < 4; r++) o[2 * (base + r) + m] = (_Float16)v[r];
+            for (int r = 0; r < 4; r++) o[2 * (base + r) + m] = (_Float16)v[b][r];
         }
-        if (NB > 1) __syncthreads();             // xs is reused by the next block's transform
     }
 }
 
@@ -302,15 +384,18 @@ __global__ __launch_bounds__(256) void k_norm_fwht(const float* __restrict__ src
 hipError_t launch_norm_fwht(const float* src, const float* src2, const float* gs, void* out, int out_dtype,
                             int out_layout, float* xnew, const float* gamma, void* hout, int flags, int W, int M,
                             int mode, hipStream_t s) {
-    // whole rows per workgroup once there are enough rows to fill the CUs (hidden width 5120);
-    // the operand form (out_dtype 2) takes M <= 8
-    if (W == 5120 && M >= 64 && out_dtype != 2)
-        hipLaunchKernelGGL(k_norm_fwht<5>, dim3(M), dim3(256), 0, s, src, src2, gs, out, out_dtype, out_layout, xnew,
-                           gamma, hout, flags, W, mode);
-    else
-        hipLaunchKernelGGL(k_norm_fwht<1>, dim3(W / 1024, M), dim3(256), 0, s, src, src2, gs, out, out_dtype,
-                           out_layout, xnew, gamma, hout, flags, W, mode);
-    return hipGetLastError();
+    auto go = [&](auto kern, dim3 grid) {
+        hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, src, src2, gs, out, out_dtype, out_layout, xnew, gamma, hout,
+                           flags, W, mode);
+        return hipGetLastError();
+    };
+    if (mode != 0) return go(k_norm_fwht<1, false>, dim3(M, W / 1024));
+    // Whole rows per workgroup read a row once, blocks per workgroup 5 times but with 5 times the
+    // waves.  Hidden width 5120, x + y to fp16, us by blocks / by rows: 64 rows 3.8 / 5.0, 96
+    // 4.1 / 5.2, 128 4.85 / 5.3, 200 8.5 / 5.6, 512 19.0 / 8.7 (by rows before the blocks shared
+    // their barriers: 6.6, 6.75, 6.9, 7.3, 9.5).  The operand form (out_dtype 2) takes M <= 8.
+    if (W == 5120 && M > 128) return go(k_norm_fwht<5, true>, dim3(M));
+    return go(k_norm_fwht<1, true>, dim3(M, W / 1024));
 }
 
 }  // namespace kata

@@ -85,3 +85,24 @@ def test_transform_feeds_the_gemv(dev):
     ref_h, _ = orc.norm_fwht(x, gs, 0)
     ref = orc.gemv_ptq1(W_np, ref_h.astype(np.float32), K, N, 1)
     assert rel_l2(y, ref).max() < 2e-3
+
+
+@pytest.mark.parametrize("W,M", [(1024, 3), (5120, 128), (5120, 129), (6144, 1), (7168, 5), (18432, 2)])
+@pytest.mark.parametrize("add", [False, True])
+def test_norm_row_splits(dev, W, M, add):
+    """Rows shorter and longer than the 6 blocks whose loads are in flight together, and both sides of
+    the line between a workgroup per block and one per row, which give the same bits."""
+    rng = np.random.default_rng(W + M)
+    x = rng.standard_normal((M, W)).astype(np.float32)
+    y = rng.standard_normal((M, W)).astype(np.float32)
+    gs, gamma = _signs(W, 4, gamma=True), (1.0 + 0.1 * rng.standard_normal(W)).astype(np.float32)
+    t = lambda a: torch.from_numpy(a).to(dev)
+    run = lambda n: ops.add_rms_fwht(t(x[:n]), t(gs), y=t(y[:n]) if add else None, gamma=t(gamma), want_xnew=True)
+    out, xnew, hout = run(M)
+    ref, href = orc.norm_fwht(x, gs, 0, src2=y if add else None, gamma=gamma, add=add)
+    # 10 + 20 levels of fp32 sums, each within 2^-24 of its terms' norm: 30 * 6e-8 = 2e-6
+    assert rel_l2(out.cpu().numpy(), ref).max() < 2e-6
+    assert rel_l2(hout.cpu().numpy(), href).max() < 2e-6
+    assert np.array_equal(xnew.cpu().numpy(), x + y if add else x)
+    for a, b in zip(run(1), (out, xnew, hout)):
+        assert torch.equal(a, b[:1])
