@@ -143,7 +143,7 @@ int kata_gemv_q8_0_batch(int count, const uint8_t* const* W, float* const* y, co
  * A is fp16 [M][lda] (lda >= K), C is [M][ldc] of c_dtype (KATA_F32 or KATA_F16).
  * K % 128 == 0; any M >= 1, N >= 1.
  * The K-pieces of the last round of tiles use a workspace of the calling (device, stream)
- * (at most one fp32 256x128 tile per CU), allocated on the first call on that stream that
+ * (at most two fp32 256x128 tiles per CU), allocated on the first call on that stream that
  * needs it and kept until kata_release_stream; a call that needs a larger buffer than the
  * stream holds must not be captured, and the outgrown buffer stays allocated (graphs captured
  * earlier may still use it).  Calls on

@@ -1,4 +1,4 @@
-// Exact fp16 prefill GEMM with the PTQ1_0 decode fused into the LDS tile load.
+// Exact fp16 prefill GEMM, the PTQ1_0 weights decoded into the MFMA's registers.
 //
 // Semantics (shaders/prefill.metal:31-41 after k_expand_ptq1_v2, :472-479):
 //   C[m][n] = sum_k A[m][k] * half(trit[n][k] * d[n][k/128]),  fp16 x fp16 -> fp32.

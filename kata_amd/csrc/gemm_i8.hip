@@ -7,14 +7,13 @@
 // gemm (shaders/prefill.metal:382-415): I = sum_{k in g} A8[m][k]*trit[n][k] (exact int32),
 //   C[m][n] = sum_g float(I) * (d[n][g] * SX[g][m]) in fp32, groups ascending.
 //
-// Design: the tile machinery of the fp16 GEMM (256 x 128 C tiles, 12 waves: 8 consumers
-// on v_mfma_i32_32x32x32_i8, two per SIMD, 4 producers copying A by DMA and decoding weights
-// into LDS, whole tiles per CU then K pieces summed by a second kernel).  A stage is one 128-group:
-// an int8 A row of 128 k is 128 bytes, the byte layout of an fp16 stage row of 64 k, so the
-// A copies, swizzle and fragment reads are the fp16 kernel's, with half the stages.  The
-// producers also stage the group's row scales (A side) and column scales (decoded weights)
-// in LDS; consumers fold each 32 x 32 tile's exact group sum into fp32 right after its
-// four MFMAs, groups ascending.
+// Two kernels.  Tall (256 x 128 C tiles): 12 waves, 8 consumers on v_mfma_i32_32x32x32_i8, two
+// per SIMD, and 4 producers that copy A by DMA and decode weights into LDS (gemm_tile.h), whole
+// tiles per CU, then K pieces summed by a second kernel.  A stage is one 128-group; the
+// producers also stage the group's row scales (A side) and column scales (decoded weights) in
+// LDS, and consumers fold each 32 x 32 tile's exact group sum into fp32 right after its four
+// MFMAs, groups ascending.  Short (32, 64 and 128 rows): every wave decodes its weights into
+// MFMA registers on the skeleton of the fp16 GEMM (gemm_reg.h); launch_gemm_i8 has the rule.
 #include "common.h"
 #include "launch.h"
 #include "gemm_ptq1_copy.h"

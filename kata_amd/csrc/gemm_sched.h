@@ -1,4 +1,5 @@
-// Tile schedule shared by the prefill GEMMs (gemm_f16.hip, gemm_i8.hip).
+// Tile schedule of the prefill GEMMs: the piece bookkeeping (gemm_job, the workspace) of all of
+// them, and the plan of the tall int8 kernel (gemm_i8.hip; the others plan in gemm_reg.h).
 //
 // C is cut into TBM x TBN tiles, tile t = (row tile t / G, column group t % G).  With
 // `slots` workgroups resident at once, the whole rounds of `slots` tiles are taken whole by
@@ -111,7 +112,7 @@ inline hipError_t launch_pieces_sum(const float* ws, void* C, int c_dtype, int l
 }
 
 // The calling thread's device: its CU count and (need_ws) the K-piece workspace of stream s
-// (room for one 256 x 128 fp32 tile per CU: 32 MB on MI355X), allocated on the first call on
+// (room for two 256 x 128 fp32 tiles per CU: 64 MB on MI355X), allocated on the first call on
 // that (device, stream) that asks for it and kept; calls on other streams use their own.
 hipError_t gemm_device(bool need_ws, hipStream_t s, int* n_cu, float** ws);
 

@@ -1,13 +1,12 @@
-// Tile machinery shared by the fp16 prefill GEMMs with a fused weight decode
-// (gemm_f16.hip: PTQ1_0, gemm_q8.hip: Q8_0).  A workgroup of 8 waves computes a
-// 256 x 128 tile of C in stages of 64 k: waves 0..3 (consumers) run v_mfma_f32_32x32x16_f16
-// on fp16 A and B tiles in LDS, waves 4..7 (producers) copy A tiles into LDS by DMA two
-// stages ahead (three A buffers) and write the decoded fp16 weights of the next stage into
-// one of two B buffers.  A stage is released by a workgroup barrier.
+// LDS tiles, copies and barriers of the tall int8 prefill GEMM (gemm_i8.hip): a workgroup of
+// producer and consumer waves computes a 256 x 128 tile of C in stages of 128 bytes of k per
+// row.  The producers copy A tiles into LDS by DMA two stages ahead (three A buffers) and write
+// the decoded weights of the next stage into one of two B buffers; a stage is released by a
+// workgroup barrier.
 //
-// LDS: [kABuf][BM rows][ROWB] A tiles, then [2][BN rows][ROWB] B tiles, then whatever the
-// producers stage (format specific).  Rows are 64 halves (128 B) of 8 chunks of 16 B; chunk
-// c of row r is stored at c ^ ((r >> 1) & 7) (conflict-free fragment reads).
+// LDS: [kABuf][BM rows][ROWB] A tiles, then [2][BN rows][ROWB] B tiles, then what the producers
+// stage besides.  Rows are 128 B in 8 chunks of 16 B; chunk c of row r is stored at
+// c ^ ((r >> 1) & 7) (conflict-free fragment reads).
 #pragma once
 #include "common.h"
 #include "gemm_sched.h"
@@ -46,91 +45,6 @@ __device__ inline uint32_t lds_addr(const void* p) {
 __device__ inline void barrier_lds() {
     __builtin_amdgcn_s_waitcnt((15 & 15) | ((63 >> 4) << 14) | (7 << 4) | (0 << 8));   // lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
-}
-
-// Consumer waves (wave < 4) of job `job`: nst stages, then the tile (or, for a piece of a
-// split tile, its fp32 partial into the job's workspace slot).  Barriers: two before the
-// first stage (the producers' first copies landed, stage 0 produced), one per stage.
-template <bool C_F16>
-__device__ inline void consume(uint8_t* smem, int wave, int lane, int nst, int job, const GemmJobs& J, float* ws,
-                               void* C, int ldc, int M, int m0, int n0, int R) {
-    auto As = [&](int buf) { return tile_a(smem, buf); };
-    auto Bs = [&](int buf) { return tile_b(smem, buf); };
-    auto barrier = [&]() { barrier_lds(); };
-    // ================= consumers =================
-    const int l32 = lane & 31, lh = lane >> 5;
-    v16f acc[2][NT];
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < NT; j++)
-#pragma unroll
-            for (int q = 0; q < 16; q++) acc[i][j][q] = 0.0f;
-    // lane l reads row / column l % 32 of each 32-row tile at k = 16 kk + 8 (l / 32) .. +7,
-    // chunk 2 kk + l / 32; every tile row of this lane has the same swizzle term
-    const int xs = (l32 >> 1) & 7;
-    const uint32_t a_row = (uint32_t)(wave * 64 + l32) * ROWB, b_row = (uint32_t)l32 * ROWB;
-    auto load_frags = [&](int st, int kk, v8h (&af)[2], v8h (&bf)[NT]) {
-        const uint32_t c = (uint32_t)(((2 * kk + lh) ^ xs) << 4);
-        const uint8_t* at = As(st % kABuf) + a_row + c;
-        const uint8_t* bt = Bs(st & 1) + b_row + c;
-#pragma unroll
-        for (int i = 0; i < 2; i++) af[i] = *(const v8h*)(at + i * 32 * ROWB);
-#pragma unroll
-        for (int j = 0; j < NT; j++) bf[j] = *(const v8h*)(bt + j * 32 * ROWB);
-    };
-    auto mfmas = [&](v8h (&af)[2], v8h (&bf)[NT]) {
-#pragma unroll
-        for (int j = 0; j < NT; j++)
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bf[j], acc[i][j], 0, 0, 0);
-    };
-    // fragments are loaded one k step ahead of the MFMAs that use them; the last step
-    // of a stage is loaded before the barrier that releases the stage's buffers
-    v8h a0[2], b0[NT], a1[2], b1[NT];
-    barrier();                               // the producers' first copies landed
-    barrier();                               // stage 0 produced
-    load_frags(0, 0, a0, b0);
-    for (int st = 0; st < nst; st++) {
-        load_frags(st, 1, a1, b1);
-        mfmas(a0, b0);
-        load_frags(st, 2, a0, b0);
-        mfmas(a1, b1);
-        load_frags(st, 3, a1, b1);
-        mfmas(a0, b0);
-        barrier();                           // stage st + 1 produced; stage st's buffers free
-        if (st + 1 < nst) load_frags(st + 1, 0, a0, b0);
-        mfmas(a1, b1);
-    }
-    // store: lane holds D[8(q/4) + 4(l/32) + q%4][l % 32] of each 32x32 tile
-    if (job >= J.n_full) {
-        // piece: the whole fp32 tile, [256][128], into the job's workspace slot
-        float* P = ws + (size_t)(job - J.n_full) * (BM * BN);
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-            for (int j = 0; j < NT; j++)
-#pragma unroll
-                for (int q = 0; q < 16; q++)
-                    P[(wave * 64 + i * 32 + 8 * (q >> 2) + 4 * lh + (q & 3)) * BN + j * 32 + l32] = acc[i][j][q];
-        return;
-    }
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < NT; j++) {
-            const int gc = j * 32 + l32;     // tile column
-            const int gn = n0 + gc;
-#pragma unroll
-            for (int q = 0; q < 16; q++) {
-                const int gm = m0 + wave * 64 + i * 32 + 8 * (q >> 2) + 4 * lh + (q & 3);
-                if (gm < M && gc < R) {
-                    if (C_F16) ((_Float16*)C)[(size_t)gm * ldc + gn] = (_Float16)acc[i][j][q];
-                    else ((float*)C)[(size_t)gm * ldc + gn] = acc[i][j][q];
-                }
-            }
-        }
 }
 
 // Producer A copies: DMA instruction i of producer pw copies LDS bytes [1024 (4i + pw), +1024)
