@@ -103,15 +103,6 @@ __device__ inline void fold_tile(v16f& acc, const v16i& I, float w, float sxv, s
     ((acc[Q] += (float)I[Q] * (w * row_bcast<Q>(sxv))), ...);
 }
 
-// LDS DMA of one dword per lane to lds + 4*lane (lds wave-uniform); see dma16
-__device__ inline void dma4(const void* g, uint32_t lds) {
-    uint32_t saved;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\tglobal_load_lds_dword %1, off\n\ts_mov_b32 m0, %0"
-                 : "=&s"(saved)
-                 : "v"(g), "s"(lds)
-                 : "memory");
-}
-
 // Consumer waves (wave < kCW): wave w owns rows 32w..32w+31 and all 128 columns, 4 tiles of
 // 32 x 32.  Per stage (one group of 128 k) the A fragments stay in registers; for each column
 // tile j the int32 sum is 4 dependent v_mfma_i32_32x32x32_i8, then folded: acc += float(I) *
@@ -454,11 +445,11 @@ __global__ __launch_bounds__(512, 2) void k_gemm_i8_short(const int8_t* __restri
         for (int i = 0; i < NA; i++) {
             const int r0 = min(m0 + i * 64, M - 1);
             const uint32_t lim = M - 1 - r0 < 64 ? (uint32_t)(M - 1 - r0) * (uint32_t)K + 112u : 0xffffffffu;
-            rg::dma16(ko + (size_t)r0 * K, min(avo, lim), a_lds + buf * C::ASTAGE + i * 8192);
+            dma16(ko + (size_t)r0 * K, min(avo, lim), a_lds + buf * C::ASTAGE + i * 8192);
         }
         // the stage's row scales, one dword per lane: wave w rows 64 (w % (SXROWS / 64)) + lane
         const int rg64 = wave & (C::SXROWS / 64 - 1);
-        rg::dma4(SX + (size_t)(kb0 + min(st, nb - 1)) * ldS, 4u * (uint32_t)min(m0 + 64 * rg64 + lane, M - 1),
+        dma4(SX + (size_t)(kb0 + min(st, nb - 1)) * ldS, 4u * (uint32_t)min(m0 + 64 * rg64 + lane, M - 1),
                  C::kSx + buf * (C::SXROWS * 4) + 256u * rg64);
     };
     Trits dec;

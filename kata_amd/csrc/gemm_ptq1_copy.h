@@ -53,7 +53,7 @@ struct Ptq1Copy {
         const uint32_t add = 2 * g + 1 == nblk ? wsingle : 0u;
 #pragma unroll
         for (int i = i0; i < i1; i++)
-            rg::dma16(wbase[i] + (size_t)g * (2 * kBlockBytes), wvo[i] + add,
+            dma16(wbase[i] + (size_t)g * (2 * kBlockBytes), wvo[i] + add,
                       w_lds + slot * slot_bytes<C>() + i * (C::THREADS * 16));
     }
 };

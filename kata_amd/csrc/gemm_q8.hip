@@ -71,7 +71,7 @@ struct Q8F16 {
 #pragma unroll
         for (int i = i0; i < i1; i++) {
             const int at = i * C::THREADS + wave * 64 < C::BN * kPieces ? i : i - 1;
-            rg::dma16(wbase + (size_t)g * 136, wvo[i],
+            dma16(wbase + (size_t)g * 136, wvo[i],
                       __builtin_amdgcn_readfirstlane(w_lds + slot * slot_bytes<C>() + at * (C::THREADS * 16)));
         }
     }

@@ -21,6 +21,7 @@
 
 #include "common.h"
 #include "gemm_sched.h"
+#include "lds_dma.h"
 
 namespace kata {
 namespace rg {
@@ -67,24 +68,6 @@ __device__ inline void unroll(F&& f) {
     unroll_impl<0, NN>(f);
 }
 
-// LDS DMA, 16 bytes per lane from base + voff to lds + 16*lane (base, lds wave-uniform).  Through
-// inline assembly so that the compiler does not make later LDS accesses wait for every copy in
-// flight; the kernel waits explicitly.  M0 is restored.
-__device__ inline void dma16(const void* base, uint32_t voff, uint32_t lds) {
-    uint32_t saved;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-                 : "=&s"(saved)
-                 : "v"(voff), "s"(base), "s"(lds)
-                 : "memory");
-}
-// the same, one dword per lane to lds + 4*lane
-__device__ inline void dma4(const void* base, uint32_t voff, uint32_t lds) {
-    uint32_t saved;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\tglobal_load_lds_dword %1, %2\n\ts_mov_b32 m0, %0"
-                 : "=&s"(saved)
-                 : "v"(voff), "s"(base), "s"(lds)
-                 : "memory");
-}
 template <int VM>
 __device__ inline void wait_vm() {
     static_assert(VM >= 0 && VM < 64, "vmcnt");

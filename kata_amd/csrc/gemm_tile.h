@@ -10,6 +10,7 @@
 #pragma once
 #include "common.h"
 #include "gemm_sched.h"
+#include "lds_dma.h"
 
 namespace kata {
 namespace gemm {
@@ -27,20 +28,6 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 __device__ inline uint32_t swz(int row, int chunk) { return (uint32_t)(row * ROWB + ((chunk ^ ((row >> 1) & 7)) << 4)); }
 __device__ inline uint8_t* tile_a(uint8_t* smem, int buf) { return smem + buf * (BM * ROWB); }
 __device__ inline uint8_t* tile_b(uint8_t* smem, int buf) { return smem + kABuf * BM * ROWB + buf * (BN * ROWB); }
-
-// LDS DMA, 16 bytes per lane to lds + 16*lane (lds wave-uniform); issued through inline
-// assembly so that the compiler does not make later LDS accesses wait for every load in
-// flight; the kernel waits for these copies explicitly.  M0 is restored.
-__device__ inline void dma16(const void* g, uint32_t lds) {
-    uint32_t saved;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
-                 : "=&s"(saved)
-                 : "v"(g), "s"(lds)
-                 : "memory");
-}
-__device__ inline uint32_t lds_addr(const void* p) {
-    return __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(__attribute__((address_space(3))) const void*)p);
-}
 
 __device__ inline void barrier_lds() {
     __builtin_amdgcn_s_waitcnt((15 & 15) | ((63 >> 4) << 14) | (7 << 4) | (0 << 8));   // lgkmcnt(0)

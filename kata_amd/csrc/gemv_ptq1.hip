@@ -31,6 +31,7 @@
 #include "common.h"
 #include "gemv_operand.h"
 #include "launch.h"
+#include "lds_dma.h"
 
 #include <algorithm>
 #include <mutex>
@@ -116,21 +117,6 @@ __host__ __device__ inline int gemv_s_lds_bytes(int nbv, int T) { return (8 * nb
 __host__ __device__ constexpr int gemv_static_lds_bytes(int LR) { return lut_bytes(LR); }
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-
-// LDS DMA of 16 bytes per lane: lane l's 16 bytes at g go to LDS byte address lds + 16*l
-// (lds wave-uniform).  Issued through inline assembly so that the compiler does not make
-// every later LDS access wait for all vector-memory loads in flight (it cannot tell which
-// LDS bytes a DMA writes); the kernel waits for these copies explicitly.  M0 is restored.
-__device__ inline void dma16(const void* g, uint32_t lds) {
-    uint32_t saved;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
-                 : "=&s"(saved)
-                 : "v"(g), "s"(lds)
-                 : "memory");
-}
-__device__ inline uint32_t lds_addr(const void* p) {
-    return __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(__attribute__((address_space(3))) const void*)p);
-}
 
 // 8 consecutive activations x[t][k0..k0+7] as floats.  Layouts: rows x[T][K] (fp16 or
 // fp32), or half2-interleaved x[K][2] fp16 (T = 2).
