@@ -14,9 +14,9 @@
 // GEMV's operand form of the fp32 values (gemv_operand.h), staged per 1024-block in LDS
 // and written as whole 16-byte A rows.
 //
-// Design: a 256-thread workgroup per (1024-block, token) for few rows (more workgroups in
-// flight; each reads the row for its sum of squares, L2-resident after the first), per
-// token row for many (the row read once, held in registers).  Element k = 4 tid + r of a
+// Design: a 256-thread workgroup per (1024-block, token) (with the norm each reads the row for its
+// sum of squares, L2-resident after the first), or per token row where that is the faster
+// (the row read once, held in registers).  Element k = 4 tid + r of a
 // block: bits 0-1 are a thread's registers, bits 2-7 its lane (butterflies by cross-lane
 // exchange), bits 8-9 its wave (one LDS transpose).  The sum of squares is reduced in a
 // fixed order: a butterfly across the wave's lanes, then the 4 waves through LDS.
@@ -162,10 +162,6 @@ __device__ inline int gdn_perm(int i) {
     return h + 128 * (k + 16 * rr);
 }
 
-// flags: 1 = add y, 2 = write xnew, 4 = write hout, 8 = hout fp16.
-// NB blocks per workgroup: NB = 1 -> grid (W/1024, M), every block's workgroup reads the
-// row for the sum of squares (few rows: more workgroups in flight); NB = W/1024 -> grid M,
-// one workgroup per row, the row read once and held in registers (many rows).
 // This workgroup's 8 blocks of token m (elements 4 tid + r of the 1024-block blk) in the
 // decode GEMV's operand form: the 32 lanes of a block reduce its amax, the limbs go to an
 // LDS copy of the 8 block images, then 128 threads store the token's 16-byte A rows.
@@ -243,22 +239,30 @@ __device__ inline void store_operand_wide(const float (&v)[4], uint2 offw, int t
     }
 }
 
-template <int NB, bool NORM>
+// flags: 2 = write xnew, 4 = write hout, 8 = hout fp16.  NORM: mode 0, ADD: of x + y.
+// ROW: grid M, a workgroup holds a row (NB = W/1024), read once.  Otherwise a workgroup holds one
+// block (NB = 1) and, with NORM, reads the rest of its row for the sum of squares.  Workgroups go
+// round robin to 8 XCDs; from 8 rows on, grid (8 W/1024, M/8) puts the blocks of row 8 y + i on XCD i
+// one after the other: the row comes once from HBM and then from that XCD's L2.  x + y, norm to fp16, us with
+// the rows or the blocks of one row consecutive / so: 333 rows of 6144 18 / 19 / 8.9, 7300 rows
+// 468 / 362 / 188, 7300 rows of 17408 3555 / 1254 / 880; SwiGLU, 7300 rows of 17408, 250 / 224 / 220.
+template <int NB, bool NORM, bool ROW, bool ADD>
 __global__ __launch_bounds__(256) void k_norm_fwht(const float* __restrict__ src, const float* __restrict__ src2,
                                                    const float* __restrict__ gs, void* __restrict__ out, int out_dtype,
                                                    int out_layout, float* __restrict__ xnew,
                                                    const float* __restrict__ gamma, void* __restrict__ hout,
-                                                   int flags, int W, int mode) {
+                                                   int flags, int W, int M, int mode) {
     __shared__ float xs[NB * 1024];
     __shared__ float part[4];
     const int tid = threadIdx.x;
-    const int m = blockIdx.x, blk0 = blockIdx.y;          // rows in x: y ends at 65535
+    const int m = ROW ? blockIdx.x : M < 8 ? blockIdx.y : 8 * blockIdx.y + (blockIdx.x & 7);
+    const int blk0 = ROW ? 0 : M < 8 ? blockIdx.x : blockIdx.x >> 3;
+    if (!ROW && m >= M) return;
     const size_t ro = (size_t)m * W;
     // the operand form's image offsets of this thread's 4 elements, loaded first (their
     // latency then overlaps the row loads)
     uint2 offw = make_uint2(0, 0);
     if (out_dtype == 2) {
-        const int M = gridDim.x;
         offw = *(const uint2*)&kOperandOff.v[M <= 2 ? M - 1 : 2][(4 * tid) & 127];
     }
     // Few rows are bound by latency: every load of the blocks and of the row's sum of squares is
@@ -277,39 +281,38 @@ __global__ __launch_bounds__(256) void k_norm_fwht(const float* __restrict__ src
     float inv = 1.0f;
     if constexpr (NORM) {
         constexpr int NR = 6;                    // 1024-blocks of the row in flight
-        const float* const yrow = (flags & 1 ? src2 : src) + ro;
-        float4 ra[NB == 1 ? NR : 1], rc[NB == 1 ? NR : 1];
-        if constexpr (NB == 1) {
+        const float* const yrow = ADD ? src2 + ro : nullptr;
+        const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+        float4 ra[ROW ? 1 : NR], rc[ROW ? 1 : NR];
+        if constexpr (!ROW) {
 #pragma unroll
             for (int j = 0; j < NR; j++) {
                 const int i = 4 * tid + (1024 * j < W ? 1024 * j : 0);
                 ra[j] = *(const float4*)(src + ro + i);
-                rc[j] = *(const float4*)(yrow + i);
+                rc[j] = ADD ? *(const float4*)(yrow + i) : zero;
             }
         }
 #pragma unroll
         for (int b = 0; b < NB; b++) {
             const int base = (blk0 + b) * 1024 + 4 * tid;
             const float4 a = *(const float4*)(src + ro + base);
-            float4 c = *(const float4*)(yrow + base);
-            if (!(flags & 1)) c = make_float4(0.f, 0.f, 0.f, 0.f);
+            const float4 c = ADD ? *(const float4*)(yrow + base) : zero;
             s[b][0] = a.x + c.x;
             s[b][1] = a.y + c.y;
             s[b][2] = a.z + c.z;
             s[b][3] = a.w + c.w;
         }
         float ss = 0.0f;
-        auto add = [&](const float4& a, float4 c) {
-            if (!(flags & 1)) c = make_float4(0.f, 0.f, 0.f, 0.f);
+        auto add = [&](const float4& a, const float4& c) {
             const float v0 = a.x + c.x, v1 = a.y + c.y, v2 = a.z + c.z, v3 = a.w + c.w;
             ss += (v0 * v0 + v1 * v1) + (v2 * v2 + v3 * v3);
         };
-        if constexpr (NB == 1) {
+        if constexpr (!ROW) {
 #pragma unroll
             for (int j = 0; j < NR; j++)
                 if (1024 * j < W) add(ra[j], rc[j]);
             for (int i = 4 * tid + 1024 * NR; i < W; i += 1024) {
-                add(*(const float4*)(src + ro + i), *(const float4*)(yrow + i));
+                add(*(const float4*)(src + ro + i), ADD ? *(const float4*)(yrow + i) : zero);
             }
         } else {
 #pragma unroll
@@ -361,7 +364,6 @@ __global__ __launch_bounds__(256) void k_norm_fwht(const float* __restrict__ src
     for (int b = 0; b < NB; b++) {
         const int base = (blk0 + b) * 1024 + 4 * tid;
         if (out_dtype == 2) {
-            const int M = gridDim.x;
             if (M <= 2)
                 store_operand(v[b], offw, tid, blk0 + b, m, M, W, (uint8_t*)xs, (uint8_t*)out);
             else
@@ -386,16 +388,24 @@ hipError_t launch_norm_fwht(const float* src, const float* src2, const float* gs
                             int mode, hipStream_t s) {
     auto go = [&](auto kern, dim3 grid) {
         hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, src, src2, gs, out, out_dtype, out_layout, xnew, gamma, hout,
-                           flags, W, mode);
+                           flags, W, M, mode);
         return hipGetLastError();
     };
-    if (mode != 0) return go(k_norm_fwht<1, false>, dim3(M, W / 1024));
-    // Whole rows per workgroup read a row once, blocks per workgroup 5 times but with 5 times the
-    // waves.  Hidden width 5120, x + y to fp16, us by blocks / by rows: 64 rows 3.8 / 5.0, 96
-    // 4.1 / 5.2, 128 4.85 / 5.3, 200 8.5 / 5.6, 512 19.0 / 8.7 (by rows before the blocks shared
-    // their barriers: 6.6, 6.75, 6.9, 7.3, 9.5).  The operand form (out_dtype 2) takes M <= 8.
-    if (W == 5120 && M > 128) return go(k_norm_fwht<5, true>, dim3(M));
-    return go(k_norm_fwht<1, true>, dim3(M, W / 1024));
+    const dim3 blocks = M < 8 ? dim3(W / 1024, M) : dim3(8 * (W / 1024), (M + 7) / 8);
+    // Without the norm nothing is shared by a row's blocks: blocks at every size (width 5120 to fp16, us
+    // by rows / by blocks: 64 rows of SwiGLU 6.9 / 3.1, 7300 75.5 / 67.4; plain 5.8 / 2.8, 39.9 / 36.6).
+    if (mode != 0) return go(k_norm_fwht<1, false, false, false>, blocks);
+    // With it, whole rows per workgroup read a row once, blocks per workgroup W/1024 times but with
+    // as many times the waves.  Width 5120, x + y to fp16, us by blocks / by rows: 64 rows 4.2 / 5.0,
+    // 129 4.9 / 5.5, 200 5.7 / 5.8, 256 6.5 / 6.1, 512 10.2 / 8.6, 7300 161 / 94.  At width 1024 the
+    // block is the row.
+    auto norm = [&](auto add) {
+        constexpr bool ADD = decltype(add)::value;
+        if (W == 1024) return go(k_norm_fwht<1, true, true, ADD>, dim3(M));
+        if (W == 5120 && M > 200) return go(k_norm_fwht<5, true, true, ADD>, dim3(M));
+        return go(k_norm_fwht<1, true, false, ADD>, blocks);
+    };
+    return flags & 1 ? norm(std::true_type{}) : norm(std::false_type{});
 }
 
 }  // namespace kata

@@ -87,7 +87,7 @@ def test_transform_feeds_the_gemv(dev):
     assert rel_l2(y, ref).max() < 2e-3
 
 
-@pytest.mark.parametrize("W,M", [(1024, 3), (5120, 128), (5120, 129), (6144, 1), (7168, 5), (18432, 2)])
+@pytest.mark.parametrize("W,M", [(1024, 3), (1024, 9), (4096, 17), (5120, 8), (5120, 200), (5120, 201), (6144, 1), (7168, 5), (18432, 2)])
 @pytest.mark.parametrize("add", [False, True])
 def test_norm_row_splits(dev, W, M, add):
     """Rows shorter and longer than the 6 blocks whose loads are in flight together, and both sides of
@@ -106,3 +106,54 @@ def test_norm_row_splits(dev, W, M, add):
     assert np.array_equal(xnew.cpu().numpy(), x + y if add else x)
     for a, b in zip(run(1), (out, xnew, hout)):
         assert torch.equal(a, b[:1])
+
+
+@pytest.mark.parametrize("mode,W", [(0, 1024), (0, 6144), (1, 17408), (2, 6144), (3, 5120)])
+@pytest.mark.parametrize("M", [7, 8, 9, 31])
+def test_rows_by_eights(dev, mode, W, M):
+    """The launch takes the rows in eights: every row of a call, whole eights or not, equals the
+    row by itself bit for bit."""
+    rng = np.random.default_rng(mode + W + M)
+    t = lambda a: torch.from_numpy(a.astype(np.float32)).to(dev)
+    src, src2, gs = t(rng.standard_normal((M, W))), t(rng.standard_normal((M, W))), t(_signs(W, 5))
+    run = lambda a, b: ops.rms_fwht(a, gs, mode, src2=b if mode == 1 else None)
+    out = run(src, src2)
+    for m in range(M):
+        assert torch.equal(out[m:m + 1], run(src[m:m + 1].contiguous(), src2[m:m + 1].contiguous())), m
+
+
+@pytest.mark.parametrize("M", [1, 2, 5])
+def test_operand_form_of_one_block(dev, M):
+    """Width 1024, a row per workgroup: the operand form gives the GEMV the bits of the fp32 rows."""
+    K, N = 1024, 200
+    rng = np.random.default_rng(M)
+    x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32)).to(dev)
+    gs = torch.from_numpy(_signs(K, 6)).to(dev)
+    W = torch.from_numpy(orc.synth_ptq1(N, K, 7)[0]).to(dev)
+    h, _, _ = ops.add_rms_fwht(x, gs)
+    q, _, _ = ops.add_rms_fwht(x, gs, out_dtype=torch.uint8)
+    if M <= 2:
+        assert torch.equal(ops.gemv_ptq1(W, q, K, N, M), ops.gemv_ptq1(W, h, K, N, M))
+    else:
+        assert torch.equal(ops.gemv_ptq1_wide(W, q, K, N, T=M), ops.gemv_ptq1_wide(W, h, K, N))
+
+
+def test_norm_reads_each_row_from_memory_once(dev):
+    """The workgroups of a row's 17 blocks run beside each other and share its reads: the norm of
+    many long rows takes 2.3 times the transform without it (8.7 to 10 times with each block's
+    workgroups a whole column of rows apart)."""
+    W, M = 17408, 7300
+    src, gs = torch.randn((M, W), device=dev), torch.ones(W, device=dev)
+
+    def us(mode):
+        ops.rms_fwht(src, gs, mode, out_dtype=torch.float16)
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(5):
+            ops.rms_fwht(src, gs, mode, out_dtype=torch.float16)
+        b.record()
+        b.synchronize()
+        return a.elapsed_time(b)
+
+    norm, plain = us(0), us(3)
+    assert norm < 5 * plain, (norm, plain)
