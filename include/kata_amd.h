@@ -142,11 +142,13 @@ int kata_gemv_q8_0_batch(int count, const uint8_t* const* W, float* const* y, co
  * C[m][n] = sum_k A[m][k] * half(trit[n][k] * d[n][k/128]), fp32 accumulation.
  * A is fp16 [M][lda] (lda >= K), C is [M][ldc] of c_dtype (KATA_F32 or KATA_F16).
  * K % 128 == 0; any M >= 1, N >= 1.
- * The K-pieces of the last round of tiles use a workspace of the calling (device, stream)
- * (at most two fp32 256x128 tiles per CU), allocated on the first call on that stream that
- * needs it and kept until kata_release_stream; a call that needs a larger buffer than the
- * stream holds must not be captured, and the outgrown buffer stays allocated (graphs captured
- * earlier may still use it).  Calls on
+ * Where tiles are split along K (all of them, or those of the last round), the pieces' partial
+ * sums use a workspace of the calling (device, stream) (two fp32 256x128 tiles per CU: 64 MB),
+ * allocated on the first call on that stream that needs it and kept until kata_release_stream.
+ * A call that cannot have it (the stream's first such call is captured, or memory is short)
+ * runs whole tiles instead: the same sums in another order, up to six times slower for few
+ * rows, and a graph keeps that schedule for its life, so a program that captures makes one
+ * eager call on the stream first.  Calls on
  * different streams use different workspaces; calls on one stream are ordered by it.  The
  * entry points that use it: kata_gemm_ptq1_f16, kata_gemm_q8_0_f16, kata_gemm_ptq1_i8 and
  * the dispatcher's prefill calls (kata_dispatch_prefill, kata_dispatch_ffn_prefill, the

@@ -587,6 +587,35 @@ hipError_t launch_cfg(const int8_t* A8, const float* SX, int ldS, const rg::Mats
 
 }  // namespace short_i8
 
+// The kernel of a call and its schedule, with K pieces or (pieces false) whole tiles only.
+constexpr int kTall = 3;             // k: of short_i8::kShapes, or the tall kernel
+struct Plan {
+    GemmJobs J;
+    int k;
+};
+// The short tiles where the cost model has them cheaper than the tall kernel's schedule (whole
+// rounds of 256 x 128 tiles at 1.3 us per group, the rest in K pieces); their row offsets are
+// 32-bit.
+Plan plan(int M, int K, int N, int n_cu, bool pieces) {
+    const int nbk = K / kGroup;
+    Plan p{plan_gemm_jobs(M, N, K, BM, BN, n_cu), kTall};   // one workgroup per CU
+    if (!pieces) {
+        const int T = p.J.n_full + (p.J.n_jobs - p.J.n_full) / p.J.S;
+        p.J = {p.J.G, T, 1, T};
+    }
+    const int rem = p.J.n_jobs - p.J.n_full;
+    double us = (p.J.n_full + n_cu - 1) / n_cu * (3.0 + nbk * 1.3);
+    if (rem) us += 3.0 + (nbk + p.J.S - 1) / p.J.S * 1.3 + 4.0 + (double)rem * BM * BN * 8.0 / 4e6;
+    for (int i = 0; i < kTall && K <= (1 << 23); i++) {
+        const rg::Plan t = rg::plan(short_i8::kShapes[i], M, (N + 255) / 256, nbk, n_cu, pieces);
+        if (t.us < us) {
+            us = t.us;
+            p = {t.J, i};
+        }
+    }
+    return p;
+}
+
 }  // namespace
 
 hipError_t launch_quant_rows(const uint16_t* X, int8_t* Q, float* SX, int M, int K, int ldS, hipStream_t s) {
@@ -611,58 +640,35 @@ hipError_t launch_gemm_i8(const int8_t* A8, const float* SX, int ldS, const uint
     float* ws = nullptr;
     hipError_t e = gemm_device(false, s, &n_cu, &ws);
     if (e != hipSuccess) return e;
-    // The short tiles where the cost model has them cheaper than the tall kernel's schedule (whole
-    // rounds of 256 x 128 tiles at 1.3 us per group, the rest in K pieces); their row offsets
-    // are 32-bit.
-    GemmJobs J = plan_gemm_jobs(M, N, K, BM, BN, n_cu);   // one workgroup per CU
-    if (K <= (1 << 23)) {
-        const int nbk = K / kGroup, G = (N + 255) / 256, rem = J.n_jobs - J.n_full;
-        auto rounds = [&](int jobs) { return (jobs + n_cu - 1) / n_cu; };
-        double tall = rounds(J.n_full) * (3.0 + nbk * 1.3);
-        if (rem) tall += 3.0 + (nbk + J.S - 1) / J.S * 1.3 + 4.0 + (double)rem * BM * BN * 8.0 / 4e6;
-        int k = -1;
-        auto choose = [&](bool pieces) {
-            rg::Plan best{};
-            for (int i = 0; i < 3; i++) {
-                const rg::Plan p = rg::plan(short_i8::kShapes[i], M, G, nbk, n_cu, pieces);
-                if (k < 0 || p.us < best.us) {
-                    best = p;
-                    k = i;
-                }
-            }
-            return best;
-        };
-        rg::Plan p = choose(true);
-        if (p.us < tall) {
-            if (p.J.n_jobs > p.J.n_full && gemm_device(true, s, &n_cu, &ws) != hipSuccess) {
-                (void)hipGetLastError();
-                k = -1;
-                p = choose(false);
-            }
-            rg::Mats P{};
-            P.W[0] = W;
-            P.C[0] = C;
-            P.N[0] = N;
-            P.ldc[0] = ldc;
-            for (int i = 1; i <= rg::kMaxMats; i++) P.g0[i] = 0x7fffffff;
-            const bool v4 = N % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)C & 15) == 0;
-            switch (k) {
-                case 0: return short_i8::launch_cfg<short_i8::Cfg<1>>(A8, SX, ldS, P, ws, c_dtype, v4, M, K, p.J, s);
-                case 1: return short_i8::launch_cfg<short_i8::Cfg<2>>(A8, SX, ldS, P, ws, c_dtype, v4, M, K, p.J, s);
-                default: return short_i8::launch_cfg<short_i8::Cfg<4>>(A8, SX, ldS, P, ws, c_dtype, v4, M, K, p.J, s);
-            }
+    Plan p = plan(M, K, N, n_cu, true);
+    if (p.J.n_jobs > p.J.n_full && gemm_device(true, s, &n_cu, &ws) != hipSuccess) {
+        // no workspace (the stream's first call is captured, or memory is short): whole tiles
+        (void)hipGetLastError();
+        p = plan(M, K, N, n_cu, false);
+    }
+    if (p.k < kTall) {
+        rg::Mats P{};
+        P.W[0] = W;
+        P.C[0] = C;
+        P.N[0] = N;
+        P.ldc[0] = ldc;
+        for (int i = 1; i <= rg::kMaxMats; i++) P.g0[i] = 0x7fffffff;
+        const bool v4 = N % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)C & 15) == 0;
+        switch (p.k) {
+            case 0: return short_i8::launch_cfg<short_i8::Cfg<1>>(A8, SX, ldS, P, ws, c_dtype, v4, M, K, p.J, s);
+            case 1: return short_i8::launch_cfg<short_i8::Cfg<2>>(A8, SX, ldS, P, ws, c_dtype, v4, M, K, p.J, s);
+            default: return short_i8::launch_cfg<short_i8::Cfg<4>>(A8, SX, ldS, P, ws, c_dtype, v4, M, K, p.J, s);
         }
     }
-    if (J.n_jobs > J.n_full && (e = gemm_device(true, s, &n_cu, &ws)) != hipSuccess) return e;
     if (c_dtype == 1)
-        hipLaunchKernelGGL(k_gemm_ptq1_i8<true>, dim3(J.n_jobs), dim3(64 * (kCW + 4)), kLdsBytes, s, A8, SX, ldS, W, C, ldc, ws,
-                           M, K, N, J);
+        hipLaunchKernelGGL(k_gemm_ptq1_i8<true>, dim3(p.J.n_jobs), dim3(64 * (kCW + 4)), kLdsBytes, s, A8, SX, ldS, W, C, ldc, ws,
+                           M, K, N, p.J);
     else
-        hipLaunchKernelGGL(k_gemm_ptq1_i8<false>, dim3(J.n_jobs), dim3(64 * (kCW + 4)), kLdsBytes, s, A8, SX, ldS, W, C, ldc,
-                           ws, M, K, N, J);
+        hipLaunchKernelGGL(k_gemm_ptq1_i8<false>, dim3(p.J.n_jobs), dim3(64 * (kCW + 4)), kLdsBytes, s, A8, SX, ldS, W, C, ldc,
+                           ws, M, K, N, p.J);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return launch_pieces_sum<BM, BN>(ws, C, c_dtype, ldc, M, N, J, s);
+    return launch_pieces_sum<BM, BN>(ws, C, c_dtype, ldc, M, N, p.J, s);
 }
 
 }  // namespace kata

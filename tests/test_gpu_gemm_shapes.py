@@ -6,11 +6,14 @@ one launch, and rows too far apart for 32-bit offsets.
 
 Reference: float64 products of the expanded weights.  Bar: fp32 sums of K fp16 products err by
 about sqrt(K) 2^-24 of their scale, at most 8e-6 at K = 17408 (1e-5 as for the other shapes)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 from kata_amd import ops
+from kata_amd.capi import check, lib
 from kata_amd.engine import Dispatch, dispatch_work_bytes
 from oracle import oracle as orc
 
@@ -93,18 +96,33 @@ def test_matrices_of_one_launch(dev, M):
                 _check(C, h, W, H, N)
 
 
-def test_first_call_captured(dev):
-    """A stream's first GEMM may be captured: without the workspace no tile is split."""
-    M, K, N = 40, 2048, 1024
-    W = _weights(dev, K, N, 40, False)
+@pytest.mark.parametrize("op,M,K,N", [("f16", 40, 2048, 1024), ("q8", 40, 2048, 1024), ("i8", 41, 5120, 1024), ("i8", 512, 5120, 5120)])
+def test_first_call_captured(dev, op, M, K, N):
+    """A stream's first GEMM may be captured: without the workspace no tile is split.  Every replay
+    gives the bits of the others and, but for the order of its sums, the eager call's result."""
     A = torch.from_numpy(orc.synth_x(M, K, 41)).to(dev)
-    C = torch.empty((M, N), device=dev)
+    if op == "q8":
+        W = torch.from_numpy(orc.synth_q8(N, K, 40)[0]).to(dev)
+        call = lambda C: ops.gemm_q8_f16(A, W, K, N, out=C)
+    else:
+        W = _weights(dev, K, N, 40, False)
+        Q, SX = ops.quant_rows(A)
+        call = (lambda C: ops.gemm_ptq1_i8(Q, SX, W, K, N, out=C)) if op == "i8" else (lambda C: ops.gemm_ptq1_f16(A, W, K, N, out=C))
+    C, eager = torch.empty((M, N), device=dev), torch.empty((M, N), device=dev)
+    call(eager)
+    torch.cuda.synchronize()
+    s = torch.cuda.Stream(dev)
+    check(lib().kata_release_stream(ctypes.c_void_p(s.cuda_stream)))    # torch reuses streams: no workspace left
     g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g, stream=torch.cuda.Stream(dev)):
-        ops.gemm_ptq1_f16(A, W, K, N, out=C)
+    with torch.cuda.graph(g, stream=s):
+        call(C)
+    first = None
     for _ in range(3):
         C.fill_(float("nan"))
         torch.cuda.synchronize()
         g.replay()
         torch.cuda.synchronize()
-        _check(C, A, W, K, N)
+        first = C.clone() if first is None else first
+        assert torch.equal(C, first)
+        err = float((C.double() - eager.double()).norm() / eager.double().norm())
+        assert err < 2e-5, err                  # two sums in fp32, each within 1e-5 of the exact one
