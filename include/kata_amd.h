@@ -166,6 +166,13 @@ int kata_gemm_ptq1_f16(const uint16_t* A, int lda, const uint8_t* W, void* C, in
 int kata_gemm_q8_0_f16(const uint16_t* A, int lda, const uint8_t* W, void* C, int c_dtype, int ldc,
                        int M, int K, int N, void* stream);
 
+/* HOST: how a prefill GEMM is cut on a device of n_cu CUs, without launching it: format 0
+ * kata_gemm_ptq1_f16 (count matrices N[0..count-1], 1..4, that share A in one launch, as the
+ * dispatcher's), 1 kata_gemm_q8_0_f16, 2 kata_gemm_ptq1_i8 (count 1); workspace 0: as without
+ * it.  plan[0..4] = rows and columns of a tile, tiles taken whole, tiles split along K, pieces of
+ * each.  For tests and tuning; no counterpart in the reference. */
+int kata_prefill_plan(int format, int M, int K, int count, const int* N, int n_cu, int workspace, int* plan);
+
 /* Activation quantisation for the int8 prefill path: per (token m, 128-group g)
  * scale = amax > 0 ? amax/127 : 1, Q = clamp(rint(x/scale), +-127), SX[g*ldS + m] = scale.
  * X fp16 [M][K] (16-byte aligned), Q int8 [M][K] (8-byte aligned), SX fp32 [K/128][ldS],

@@ -43,6 +43,7 @@ SIGNATURES = {
     "kata_dispatch_gemv_q8": (I, [P, I, P, P, I, P, P, I, I, P]),
     "kata_gemm_ptq1_f16": (I, [P, I, P, P, I, I, I, I, I, P]),
     "kata_gemm_q8_0_f16": (I, [P, I, P, P, I, I, I, I, I, P]),
+    "kata_prefill_plan": (I, [I, I, I, I, P, I, I, P]),
     "kata_quant_rows_i8": (I, [P, P, P, I, I, I, P]),
     "kata_gemm_ptq1_i8": (I, [P, P, I, P, P, I, I, I, I, I, P]),
     "kata_expand_ptq1_f16": (I, [P, P, I, I, P]),

@@ -254,6 +254,22 @@ int kata_gemm_q8_0_f16(const uint16_t* A, int lda, const uint8_t* W, void* C, in
                         "gemm q8_0 f16");
 }
 
+int kata_prefill_plan(int format, int M, int K, int count, const int* N, int n_cu, int workspace, int* plan) {
+    if (!N || !plan) return fail(KATA_EINVAL, "null pointer argument");
+    if (format < 0 || format > 2) return fail(KATA_EINVAL, "format=%d", format);
+    if (count < 1 || count > (format == 0 ? 4 : 1)) return fail(KATA_EINVAL, "count=%d out of range", count);
+    if (M <= 0 || n_cu <= 0 || K <= 0 || K % 128 != 0) return fail(KATA_EINVAL, "bad shape M=%d K=%d n_cu=%d", M, K, n_cu);
+    for (int i = 0; i < count; i++)
+        if (N[i] <= 0) return fail(KATA_EINVAL, "N[%d]=%d must be positive", i, N[i]);
+    const kata::PrefillPlan p = format == 0   ? kata::plan_gemm_f16(M, K, count, N, n_cu, workspace != 0)
+                                : format == 1 ? kata::plan_gemm_q8(M, K, N[0], n_cu, workspace != 0)
+                                              : kata::plan_gemm_i8(M, K, N[0], n_cu, workspace != 0);
+    const int v[5] = {p.tile_rows, p.tile_cols, p.whole, p.split, p.pieces};
+    std::copy(v, v + 5, plan);
+    g_err.clear();
+    return KATA_OK;
+}
+
 int kata_quant_rows_i8(const uint16_t* X, int8_t* Q, float* SX, int M, int K, int ldS, void* stream) {
     if (!X || !Q || !SX) return fail(KATA_EINVAL, "null pointer argument");
     if (M <= 0) return fail(KATA_EINVAL, "M=%d must be positive", M);

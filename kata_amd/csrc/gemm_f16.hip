@@ -184,6 +184,10 @@ hipError_t gemm_device(bool need_ws, hipStream_t s, int* n_cu, float** ws) {
     return e;
 }
 
+PrefillPlan plan_gemm_f16(int M, int K, int count, const int* N, int n_cu, bool pieces) {
+    return rg::prefill_plan(kShapes, M, K, count, N, n_cu, pieces);
+}
+
 hipError_t launch_gemm_f16_multi(const uint16_t* A, int lda, int count, const uint8_t* const* W, void* const* C, int c_dtype,
                                  const int* ldc, int M, int K, const int* N, hipStream_t s) {
     return rg::launch<Ptq1F16, Cfg32, Cfg64, Cfg128, Cfg256>(kShapes, (const _Float16*)A, lda, count, W, C, c_dtype, ldc, M, K, N, s);

@@ -587,33 +587,26 @@ hipError_t launch_cfg(const int8_t* A8, const float* SX, int ldS, const rg::Mats
 
 }  // namespace short_i8
 
-// The kernel of a call and its schedule, with K pieces or (pieces false) whole tiles only.
-constexpr int kTall = 3;             // k: of short_i8::kShapes, or the tall kernel
-struct Plan {
-    GemmJobs J;
-    int k;
-};
-// The short tiles where the cost model has them cheaper than the tall kernel's schedule (whole
-// rounds of 256 x 128 tiles at 1.3 us per group, the rest in K pieces); their row offsets are
-// 32-bit.
-Plan plan(int M, int K, int N, int n_cu, bool pieces) {
+// The kernel of a call (k: of short_i8::kShapes, or kTall) and its schedule, with K pieces or
+// (pieces false) whole tiles only: the short tiles where the cost model has them cheaper than
+// the tall kernel's schedule (whole rounds of 256 x 128 tiles at 1.3 us per group, the rest in K
+// pieces); their row offsets are 32-bit.
+constexpr int kTall = 3;
+rg::Plan plan(int M, int K, int N, int n_cu, bool pieces) {
     const int nbk = K / kGroup;
-    Plan p{plan_gemm_jobs(M, N, K, BM, BN, n_cu), kTall};   // one workgroup per CU
+    GemmJobs J = plan_gemm_jobs(M, N, K, BM, BN, n_cu);   // one workgroup per CU
     if (!pieces) {
-        const int T = p.J.n_full + (p.J.n_jobs - p.J.n_full) / p.J.S;
-        p.J = {p.J.G, T, 1, T};
+        const int T = J.n_full + (J.n_jobs - J.n_full) / J.S;
+        J = {J.G, T, 1, T};
     }
-    const int rem = p.J.n_jobs - p.J.n_full;
-    double us = (p.J.n_full + n_cu - 1) / n_cu * (3.0 + nbk * 1.3);
-    if (rem) us += 3.0 + (nbk + p.J.S - 1) / p.J.S * 1.3 + 4.0 + (double)rem * BM * BN * 8.0 / 4e6;
-    for (int i = 0; i < kTall && K <= (1 << 23); i++) {
-        const rg::Plan t = rg::plan(short_i8::kShapes[i], M, (N + 255) / 256, nbk, n_cu, pieces);
-        if (t.us < us) {
-            us = t.us;
-            p = {t.J, i};
-        }
+    const int rem = J.n_jobs - J.n_full;
+    double us = (J.n_full + n_cu - 1) / n_cu * (3.0 + nbk * 1.3);
+    if (rem) us += 3.0 + (nbk + J.S - 1) / J.S * 1.3 + 4.0 + (double)rem * BM * BN * 8.0 / 4e6;
+    if (K <= (1 << 23)) {
+        const rg::Plan t = rg::choose(short_i8::kShapes, M, (N + 255) / 256, nbk, n_cu, pieces);
+        if (t.us < us) return t;
     }
-    return p;
+    return {J, (float)us, kTall};
 }
 
 }  // namespace
@@ -623,6 +616,12 @@ hipError_t launch_quant_rows(const uint16_t* X, int8_t* Q, float* SX, int M, int
     hipLaunchKernelGGL(k_quant_rows, dim3((unsigned)((groups + 15) / 16)), dim3(256), 0, s, (const _Float16*)X, Q, SX,
                        M, K, ldS);
     return hipGetLastError();
+}
+
+PrefillPlan plan_gemm_i8(int M, int K, int N, int n_cu, bool pieces) {
+    const rg::Plan p = plan(M, K, N, n_cu, pieces);
+    return p.k == kTall ? rg::prefill_plan(p.J, BM, BN)
+                        : rg::prefill_plan(p.J, short_i8::kShapes[p.k].bm, short_i8::kShapes[p.k].bn);
 }
 
 hipError_t launch_gemm_i8(const int8_t* A8, const float* SX, int ldS, const uint8_t* W, void* C, int c_dtype,
@@ -640,7 +639,7 @@ hipError_t launch_gemm_i8(const int8_t* A8, const float* SX, int ldS, const uint
     float* ws = nullptr;
     hipError_t e = gemm_device(false, s, &n_cu, &ws);
     if (e != hipSuccess) return e;
-    Plan p = plan(M, K, N, n_cu, true);
+    rg::Plan p = plan(M, K, N, n_cu, true);
     if (p.J.n_jobs > p.J.n_full && gemm_device(true, s, &n_cu, &ws) != hipSuccess) {
         // no workspace (the stream's first call is captured, or memory is short): whole tiles
         (void)hipGetLastError();

@@ -124,6 +124,10 @@ constexpr rg::Shape kShapes[3] = {{64, 256, 1.5f, 1.55f, 2}, {128, 256, 1.85f, 1
 
 }  // namespace
 
+PrefillPlan plan_gemm_q8(int M, int K, int N, int n_cu, bool pieces) {
+    return rg::prefill_plan(kShapes, M, K, 1, &N, n_cu, pieces);
+}
+
 hipError_t launch_gemm_q8(const uint16_t* A, int lda, const uint8_t* W, void* C, int c_dtype, int ldc, int M, int K,
                           int N, hipStream_t s) {
     return rg::launch<Q8F16, Cfg64, Cfg128, Cfg256>(kShapes, (const _Float16*)A, lda, 1, &W, &C, c_dtype, &ldc, M, K, &N, s);

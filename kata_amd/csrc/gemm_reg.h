@@ -21,6 +21,7 @@
 
 #include "common.h"
 #include "gemm_sched.h"
+#include "launch.h"
 #include "lds_dma.h"
 
 namespace kata {
@@ -358,6 +359,7 @@ struct Shape {
 struct Plan {
     GemmJobs J;
     float us;
+    int k;               // configuration
 };
 constexpr int kPieceFloats = 2 * 256 * 128;               // workspace floats per CU
 // The cheapest schedule of T = row tiles x column groups tiles on n_cu workgroups: whole tiles
@@ -371,17 +373,40 @@ inline Plan plan(const Shape& c, int M, int G, int nbk, int n_cu, bool pieces) {
         const double busy = (double)jobs / (double)(rounds * n_cu);
         return rounds * (3.0 + blocks * std::max((double)c.t_alone, c.t_full * busy));
     };
-    Plan best{{G, (int)T, 1, (int)T}, (float)part(T, nbk)};
+    Plan best{{G, (int)T, 1, (int)T}, (float)part(T, nbk), 0};
     if (!pieces) return best;
     for (long rem : {T % n_cu, T}) {
         for (int S = 2; rem && S <= kMaxPieces && S * (rem == T ? c.min_blocks : 1) <= nbk; S++) {
             if ((double)rem * S * c.bm * c.bn > (double)n_cu * kPieceFloats) break;
             const double us = (T > rem ? part(T - rem, nbk) : 0.0) + part(rem * S, (nbk + S - 1) / S) + 4.0 +
                               rem * S * rows * c.bn * 8.0 / 4e6;
-            if (us < best.us) best = {{G, (int)(T - rem), S, (int)(T - rem + rem * S)}, (float)us};
+            if (us < best.us) best = {{G, (int)(T - rem), S, (int)(T - rem + rem * S)}, (float)us, 0};
         }
     }
     return best;
+}
+
+// the cheapest of `shapes`, the first of equal ones
+template <size_t kShapes>
+inline Plan choose(const Shape (&shapes)[kShapes], int M, int G, int nbk, int n_cu, bool pieces) {
+    Plan best{};
+    for (int i = 0; i < (int)kShapes; i++) {
+        Plan p = plan(shapes[i], M, G, nbk, n_cu, pieces);
+        p.k = i;
+        if (i == 0 || p.us < best.us) best = p;
+    }
+    return best;
+}
+inline PrefillPlan prefill_plan(const GemmJobs& J, int bm, int bn) {
+    return {bm, bn, J.n_full, (J.n_jobs - J.n_full) / J.S, J.S};
+}
+// launch's plan of matrices N[0 .. count-1]
+template <size_t kShapes>
+inline PrefillPlan prefill_plan(const Shape (&shapes)[kShapes], int M, int K, int count, const int* N, int n_cu, bool pieces) {
+    int G = 0;
+    for (int i = 0; i < count; i++) G += (N[i] + shapes[0].bn - 1) / shapes[0].bn;
+    const Plan p = choose(shapes, M, G, K / 128, n_cu, pieces);
+    return prefill_plan(p.J, shapes[p.k].bm, shapes[p.k].bn);
 }
 
 template <class D, class C, bool C_F16>
@@ -463,26 +488,14 @@ hipError_t launch(const Shape (&shapes)[sizeof...(Cs)], const _Float16* A, int l
         v4 &= N[i] % 4 == 0 && ldc[i] % 4 == 0 && ((uintptr_t)C[i] & 15) == 0;
     }
     P.g0[kMaxMats] = 0x7fffffff;
-    int k = 0;
-    auto choose = [&](bool pieces) {
-        Plan best{};
-        for (int i = 0; i < kShapes; i++) {
-            const Plan p = plan(shapes[i], M, G, K / 128, n_cu, pieces);
-            if (i == 0 || p.us < best.us) {
-                best = p;
-                k = i;
-            }
-        }
-        return best.J;
-    };
-    GemmJobs J = choose(true);
-    if (J.n_jobs > J.n_full && gemm_device(true, s, &n_cu, &ws) != hipSuccess) {
+    Plan p = choose(shapes, M, G, K / 128, n_cu, true);
+    if (p.J.n_jobs > p.J.n_full && gemm_device(true, s, &n_cu, &ws) != hipSuccess) {
         // no workspace (the stream's first call is captured, or memory is short): whole tiles
         (void)hipGetLastError();
-        J = choose(false);
+        p = choose(shapes, M, G, K / 128, n_cu, false);
     }
     int i = 0;
-    ((i++ == k ? (void)(e = launch_cfg<D, Cs>(A, lda, P, ws, c_dtype, v4, M, K, J, s)) : (void)0), ...);
+    ((i++ == p.k ? (void)(e = launch_cfg<D, Cs>(A, lda, P, ws, c_dtype, v4, M, K, p.J, s)) : (void)0), ...);
     return e;
 }
 

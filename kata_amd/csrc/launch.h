@@ -49,6 +49,15 @@ hipError_t launch_gemm_f16(const uint16_t* A, int lda, const uint8_t* W, void* C
 // the same for 1..4 matrices sharing A, one launch
 hipError_t launch_gemm_f16_multi(const uint16_t* A, int lda, int count, const uint8_t* const* W, void* const* C,
                                  int c_dtype, const int* ldc, int M, int K, const int* N, hipStream_t s);
+// how a prefill GEMM would be cut on n_cu CUs (host only; pieces false: without the workspace)
+struct PrefillPlan {
+    int tile_rows, tile_cols;
+    int whole, split;    // tiles taken whole, tiles cut along K
+    int pieces;          // of each split tile
+};
+PrefillPlan plan_gemm_f16(int M, int K, int count, const int* N, int n_cu, bool pieces);
+PrefillPlan plan_gemm_q8(int M, int K, int N, int n_cu, bool pieces);
+PrefillPlan plan_gemm_i8(int M, int K, int N, int n_cu, bool pieces);
 hipError_t launch_gemm_q8(const uint16_t* A, int lda, const uint8_t* W, void* C, int c_dtype, int ldc, int M, int K,
                           int N, hipStream_t s);
 hipError_t launch_quant_rows(const uint16_t* X, int8_t* Q, float* SX, int M, int K, int ldS,

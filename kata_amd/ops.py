@@ -4,6 +4,7 @@ current stream, and raises KataError on a bad argument — there is no CPU fallb
 """
 from __future__ import annotations
 
+import collections
 import ctypes
 
 import numpy as np
@@ -228,6 +229,19 @@ def gemm_q8_f16(A: torch.Tensor, W: torch.Tensor, K: int, N: int, out_dtype=torc
     cdt = KATA_F16 if C.dtype == torch.float16 else KATA_F32
     check(lib().kata_gemm_q8_0_f16(_ptr(A), A.shape[1], _ptr(W), _ptr(C), cdt, C.shape[1], M, K, N, _stream(A)))
     return C
+
+
+PrefillPlan = collections.namedtuple("PrefillPlan", "tile_rows tile_cols whole split pieces")
+
+
+def prefill_plan(fmt: str, M: int, K: int, Ns, n_cu: int = 256, workspace: bool = True) -> PrefillPlan:
+    """How a prefill GEMM ("f16": 1..4 matrices of one launch, "q8" or "i8") would be cut on n_cu CUs:
+    tile size, tiles taken whole, tiles split along K and the pieces of each.  No GPU is used."""
+    Ns = list(Ns) if isinstance(Ns, (list, tuple)) else [Ns]
+    out = (ctypes.c_int * 5)()
+    check(lib().kata_prefill_plan(("f16", "q8", "i8").index(fmt), M, K, len(Ns), (ctypes.c_int * len(Ns))(*Ns), n_cu,
+                                  int(workspace), out))
+    return PrefillPlan(*out)
 
 
 def quant_rows(X: torch.Tensor, ldS: int | None = None, out=None):
