@@ -563,7 +563,7 @@ __global__ __launch_bounds__(512, 2) void k_gemm_i8_short(const int8_t* __restri
 }
 
 // us per 128-group of a tile (see rg::Shape), fitted to 28..2500 rows of three model shapes
-constexpr rg::Shape kShapes[3] = {{32, 256, 1.1f, 1.1f, 2}, {64, 256, 1.3f, 1.3f, 2}, {128, 256, 1.75f, 1.8f, 2}};
+constexpr rg::Shape kShapes[3] = {{32, 256, 1.1f, 1.1f, 1.0f}, {64, 256, 1.3f, 1.3f, 1.0f}, {128, 256, 1.75f, 1.8f, 1.0f}};
 
 template <class C>
 hipError_t launch_cfg(const int8_t* A8, const float* SX, int ldS, const rg::Mats& P, float* ws, int c_dtype, bool v4, int M,

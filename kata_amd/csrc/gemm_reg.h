@@ -354,7 +354,7 @@ inline hipError_t launch_pieces_sum(const float* ws, const Mats& P, int c_dtype,
 struct Shape {
     int bm, bn;
     float t_alone, t_full;
-    int min_blocks;      // of a piece where every tile is split
+    float short_gain;    // all of a table alike, see choose
 };
 struct Plan {
     GemmJobs J;
@@ -365,7 +365,8 @@ constexpr int kPieceFloats = 2 * 256 * 128;               // workspace floats pe
 // The cheapest schedule of T = row tiles x column groups tiles on n_cu workgroups: whole tiles
 // for the full rounds and the rest split S ways, or every tile split; a split costs the
 // pieces' way through memory and back (4 TB/s) and a launch (4 us); a round starts in 3 us.
-inline Plan plan(const Shape& c, int M, int G, int nbk, int n_cu, bool pieces) {
+// Where every tile is split, pieces have at least min_blocks blocks.
+inline Plan plan(const Shape& c, int M, int G, int nbk, int n_cu, bool pieces, int min_blocks) {
     const long T = (long)((M + c.bm - 1) / c.bm) * G;
     const double rows = (double)M / ((M + c.bm - 1) / c.bm);                // real rows per tile
     auto part = [&](long jobs, int blocks) {                                // a set of equal jobs
@@ -376,7 +377,7 @@ inline Plan plan(const Shape& c, int M, int G, int nbk, int n_cu, bool pieces) {
     Plan best{{G, (int)T, 1, (int)T}, (float)part(T, nbk), 0};
     if (!pieces) return best;
     for (long rem : {T % n_cu, T}) {
-        for (int S = 2; rem && S <= kMaxPieces && S * (rem == T ? c.min_blocks : 1) <= nbk; S++) {
+        for (int S = 2; rem && S <= kMaxPieces && S * (rem == T ? min_blocks : 1) <= nbk; S++) {
             if ((double)rem * S * c.bm * c.bn > (double)n_cu * kPieceFloats) break;
             const double us = (T > rem ? part(T - rem, nbk) : 0.0) + part(rem * S, (nbk + S - 1) / S) + 4.0 +
                               rem * S * rows * c.bn * 8.0 / 4e6;
@@ -386,16 +387,22 @@ inline Plan plan(const Shape& c, int M, int G, int nbk, int n_cu, bool pieces) {
     return best;
 }
 
-// the cheapest of `shapes`, the first of equal ones
+// The cheapest of `shapes`, the first of equal ones.  The model flatters pieces of a few blocks (each
+// starts and ends its own way through memory), so a schedule with pieces of 2 to 7 blocks is
+// taken only where the model has it below short_gain of the best without.
 template <size_t kShapes>
 inline Plan choose(const Shape (&shapes)[kShapes], int M, int G, int nbk, int n_cu, bool pieces) {
-    Plan best{};
-    for (int i = 0; i < (int)kShapes; i++) {
-        Plan p = plan(shapes[i], M, G, nbk, n_cu, pieces);
-        p.k = i;
-        if (i == 0 || p.us < best.us) best = p;
-    }
-    return best;
+    auto cheapest = [&](int min_blocks) {
+        Plan best{};
+        for (int i = 0; i < (int)kShapes; i++) {
+            Plan p = plan(shapes[i], M, G, nbk, n_cu, pieces, min_blocks);
+            p.k = i;
+            if (i == 0 || p.us < best.us) best = p;
+        }
+        return best;
+    };
+    const Plan any = cheapest(2), sure = cheapest(8);
+    return any.us <= shapes[0].short_gain * sure.us ? any : sure;
 }
 inline PrefillPlan prefill_plan(const GemmJobs& J, int bm, int bn) {
     return {bm, bn, J.n_full, (J.n_jobs - J.n_full) / J.S, J.S};

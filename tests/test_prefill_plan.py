@@ -1,4 +1,4 @@
-"""How the prefill GEMMs are cut (host code): tiles, K pieces, and the workspace the pieces need."""
+"""How the prefill GEMMs are cut (host code): tiles, K pieces, the workspace the pieces need."""
 import itertools
 import random
 
@@ -29,3 +29,12 @@ def test_plans_hold(fmt):
         assert (1 < p.pieces <= min(16, K // 128)) if p.split else p.pieces == 1, (M, K, Ns, p)
         assert p.split * p.pieces * p.tile_rows * p.tile_cols <= n_cu * WS_FLOATS, (M, K, Ns, p)
         assert ops.prefill_plan(fmt, M, K, Ns, n_cu, workspace=False).split == 0
+
+
+@pytest.mark.parametrize("M,K,N,shorter", [(25, 1920, 1500, True), (41, 1024, 1024, True), (41, 1920, 5000, True),
+                                           (25, 5120, 1024, True), (64, 4096, 4096, False), (100, 5120, 12288, False)])
+def test_f16_pieces_follow_time(M, K, N, shorter):
+    """Few tiles of short rows are split into pieces below 8 blocks (measured 1.3 to 1.9 times faster
+    than without); where that measured equal or slower, 8 blocks are the least."""
+    p = ops.prefill_plan("f16", M, K, N)
+    assert p.split and (K // 128 / p.pieces < 8) == shorter, p
