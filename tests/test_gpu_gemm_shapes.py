@@ -2,7 +2,8 @@
 the edges of the 32, 64, 128 and 256 row tiles, columns around the 256 column tiles, odd and
 even numbers of 128-k blocks (the packed weights are copied two blocks at a time), K splits of
 all tiles and of the last round, scales of 1 and more (another decode form), several matrices in
-one launch, and rows too far apart for 32-bit offsets.
+one launch, rows too far apart for 32-bit offsets, weight rows too long for them.  Where a test
+means a tile height or a split it asks the planner, so that a shape that no longer takes it fails.
 
 Reference: float64 products of the expanded weights.  Bar: fp32 sums of K fp16 products err by
 about sqrt(K) 2^-24 of their scale, at most 8e-6 at K = 17408 (1e-5 as for the other shapes)."""
@@ -49,14 +50,71 @@ def test_tile_edges(dev, M, K, N, big):
     _check(ops.gemm_ptq1_f16(A, W, K, N), A, W, K, N)
 
 
-@pytest.mark.parametrize("M,K,N", [(1024, 1024, 17000), (4500, 640, 5000), (2000, 5120, 1024)])
-def test_schedules(dev, M, K, N):
-    """Whole rounds with a split rest, and every tile split, at sizes of the larger tiles."""
-    W = _weights(dev, K, N, M + K, False)
+def _plan_is(dev, fmt, M, K, N, rows, kind):
+    p = ops.prefill_plan(fmt, M, K, N, torch.cuda.get_device_properties(dev).multi_processor_count)
+    assert p.tile_rows == rows and (p.whole > 0, p.split > 0) == {"whole": (True, False), "split": (False, True), "both": (True, True)}[kind], p
+
+
+def _device_weights(dev, K, N, seed, late):
+    """Weights made on the GPU; late: in every other 32 columns each third block from block 2 on
+    has a scale of 1 and more, so those waves change the decode form inside their piece."""
+    g = torch.Generator(device=dev).manual_seed(seed)
+    W = torch.randint(0, 256, (N, K // 128, 28), generator=g, device=dev, dtype=torch.uint8)
+    d = (0.02 * torch.randn((N, K // 128), generator=g, device=dev)).abs()
+    if late:
+        d[(torch.arange(N, device=dev) // 32) % 2 == 1, 2::3] *= 5000.0
+    W[:, :, 26:] = d.half().view(torch.uint8).view(N, -1, 2)
+    return W.view(N, -1)
+
+
+@pytest.mark.parametrize("late", [False, True])
+@pytest.mark.parametrize("rows,kind,M,K,N", [
+    (32, "split", 1, 1152, 257), (64, "whole", 1000, 384, 2050), (64, "split", 513, 3968, 257),
+    (64, "both", 700, 3968, 12001), (128, "whole", 513, 384, 8003), (128, "split", 600, 3968, 2050),
+    (128, "both", 1000, 5120, 9000), (256, "whole", 400, 384, 17001), (256, "both", 1000, 5120, 17001)])
+def test_tile_heights(dev, rows, kind, M, K, N, late):
+    """Every tile height with whole tiles, all tiles split and a split rest, rows and columns ragged,
+    even and odd numbers of blocks; every column by itself, so small ones count beside large, in
+    units of the norm that a column of such products has (a lone sum may come out near zero)."""
+    _plan_is(dev, "f16", M, K, N, rows, kind)
+    W = _device_weights(dev, K, N, M + K, late)
     A = torch.from_numpy(orc.synth_x(M, K, M + 6)).to(dev)
     C = ops.gemm_ptq1_f16(A, W, K, N)
-    _check(C, A, W, K, N)
+    w = ops.expand_f16(W, K, N).double()
+    err = (C.double() - A.double() @ w.t()).norm(dim=0) / (A.double().norm() * w.norm(dim=1) / K ** 0.5)
+    assert float(err.max()) < 1e-5, float(err.max())
     assert torch.equal(ops.gemm_ptq1_f16(A, W, K, N, out_dtype=torch.float16), C.half())
+
+
+@pytest.mark.parametrize("op", ["f16", "q8"])
+def test_rows_far_apart(dev, op):
+    """Rows more than 2^24 elements apart go one by one: the bits of each row's own call."""
+    M, K, N, lda = 3, 640, 300, (1 << 24) + 8
+    A = torch.zeros((M, lda), dtype=torch.float16, device=dev)
+    A[:, :K] = torch.from_numpy(orc.synth_x(M, K, 11)).to(dev)
+    W = _weights(dev, K, N, 12, True) if op == "f16" else torch.from_numpy(orc.synth_q8(N, K, 12)[0]).to(dev)
+    gemm = ops.gemm_ptq1_f16 if op == "f16" else ops.gemm_q8_f16
+    C = gemm(A, W, K, N)
+    for m in range(M):
+        assert torch.equal(C[m:m + 1], gemm(A[m:m + 1, :K].contiguous(), W, K, N)), m
+
+
+def test_long_weight_rows(dev):
+    """Weight rows of 2^24 bytes and more (256 of them span 4 GiB) go 255 columns at a time: the bits
+    of those columns' own calls.  Against float64 sums of 7.7e7 products: a single wrong 128-block
+    of a row would show as 1.1e-3 = 1 / sqrt(K / 128) and more, the roundings of the 3e5 adds of each
+    piece as 1.3e-4; the bar lies between them."""
+    K, N = 128 * 599187, 257
+    W = _device_weights(dev, K, N, 13, False)
+    assert W.shape[1] * 256 > 0xffffffff >= W.shape[1] * 255
+    A = torch.randn((1, K), generator=torch.Generator(device=dev).manual_seed(14), device=dev).half()
+    C = ops.gemm_ptq1_f16(A, W, K, N)
+    for a, b in ((0, 255), (255, 257)):
+        assert torch.equal(C[:, a:b], ops.gemm_ptq1_f16(A, W[a:b], K, b - a))
+    cols = [0, 7, 254, 255, 256]
+    ref = torch.stack([A[0].double() @ ops.expand_f16(W[n:n + 1], K, 1)[0].double() for n in cols])
+    err = float((C[0, cols].double() - ref).norm() / ref.norm())
+    assert err < 5e-4, err
 
 
 def test_strided_and_unaligned(dev):

@@ -89,9 +89,10 @@ def test_graph_long_matrix_strided_and_argmax(dev):
 
 
 def test_graph_prefill_gemm_with_pieces(dev):
-    """The fp16 prefill GEMM whose last tile round is split into K pieces (the stream's
-    workspace and the piece-sum launch) inside a graph."""
-    M, K, N = 300, 2048, 4000
+    """The fp16 prefill GEMM whose tiles are split into K pieces (the stream's workspace and the
+    piece-sum launch) inside a graph."""
+    M, K, N = 41, 6144, 5120
+    assert ops.prefill_plan("f16", M, K, N, torch.cuda.get_device_properties(dev).multi_processor_count).split
     W = torch.from_numpy(orc.synth_ptq1(N, K, 50)[0]).to(dev)
     A = torch.from_numpy(orc.synth_x(M, K, 51)).to(dev)
     C = torch.empty((M, N), dtype=torch.float16, device=dev)

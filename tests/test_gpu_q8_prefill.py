@@ -119,17 +119,24 @@ def test_gemm_f16_tile_schedules(dev):
     """Whole-tile rounds, split tiles (pieces summed from the workspace) and both together,
     called back to back so the workspace is reused with a different piece count; every
     output vs torch fp32 on the bit-exact expanded weights."""
-    cases = [(256, 128, 128 * 256),      # 256 tiles: whole tiles only (one round on 256 CUs)
-             (256, 256, 128 * 257 - 5),  # one round + 1 split tile of 2 pieces, ragged N
-             (70, 1280, 200),            # 2 tiles split 10 ways
-             (513, 384, 130)]            # 3 x 2 tiles, 3 pieces, ragged M and N
-    for M, K, N in cases:
+    cases = [(256, 128, 128 * 256, "whole"),
+             (700, 3968, 12001, "both"),   # two rounds + 5 tiles of 16 pieces, ragged M and N
+             (41, 6144, 5120, "split"),    # 40 tiles of 6 pieces
+             (1, 1152, 257, "split"),      # 2 tiles of 3 pieces
+             (70, 1280, 200, "split")]
+    n_cu = torch.cuda.get_device_properties(dev).multi_processor_count
+    seen = set()
+    for M, K, N, kind in cases:
+        p = ops.prefill_plan("f16", M, K, N, n_cu)
+        assert (p.whole > 0, p.split > 0) == {"whole": (True, False), "split": (False, True), "both": (True, True)}[kind], p
+        seen.add(p.pieces)
         W_np, _, _ = orc.synth_ptq1(N, K, M * 7 + K + N)
         A = torch.from_numpy(orc.synth_x(M, K, M + 3)).to(dev)
         W = torch.from_numpy(W_np).to(dev)
         C = ops.gemm_ptq1_f16(A, W, K, N)
         ref = A.float() @ ops.expand_f16(W, K, N).float().T
         assert rel_l2(C.cpu().numpy(), ref.cpu().numpy()).max() < 5e-5, (M, K, N)
+    assert len(seen) >= 4, seen
 
 
 @pytest.mark.parametrize("M", [1024, 7300])

@@ -29,7 +29,9 @@ def _two_streams(dev, fn, args_a, args_b, reps=4):
 
 
 def test_gemm_pieces_two_streams(dev):
-    M, K, N = 512, 1024, 17408                           # 272 tiles: the last 16 split along K
+    M, K, N = 512, 5120, 17408                           # 272 tiles: the last 16 split along K
+    p = ops.prefill_plan("f16", M, K, N, torch.cuda.get_device_properties(dev).multi_processor_count)
+    assert p.whole and p.split, p
     W = torch.from_numpy(orc.synth_ptq1(N, K, 61)[0]).to(dev)
     A1 = torch.from_numpy(orc.synth_x(M, K, 62)).to(dev)
     A2 = torch.from_numpy(orc.synth_x(M, K, 63)).to(dev)
