@@ -10,9 +10,9 @@
 //   mode 3: u = src * gs
 //   out[block b][j] = (1/32) sum_k (-1)^popcount(j & k) u[1024 b + k]
 // fp32 arithmetic; out fp32 or fp16, rows [M][W] or (M = 2) the two tokens interleaved
-// per element, [W][2] (the half2 operand of the T = 2 verify GEMV), or (M <= 2) the decode
-// GEMV's operand form of the fp32 values (gemv_operand.h), staged per 1024-block in LDS
-// and written as whole 16-byte A rows.
+// per element, [W][2] (the half2 operand of the T = 2 verify GEMV), or (M <= 2 decode, M <= 8
+// wide) the GEMV's operand form of the fp32 values (gemv_operand.h), staged per 1024-block in
+// LDS and written as whole 16-byte A rows.
 //
 // Design: a 256-thread workgroup per (1024-block, token) (with the norm each reads the row for its
 // sum of squares, L2-resident after the first), or per token row where that is the faster
@@ -261,9 +261,9 @@ __global__ __launch_bounds__(256) void k_norm_fwht(const float* __restrict__ src
     const size_t ro = (size_t)m * W;
     // the operand form's image offsets of this thread's 4 elements, loaded first (their
     // latency then overlaps the row loads)
-    uint2 offw = make_uint2(0, 0);
-    if (out_dtype == 2) {
-        offw = *(const uint2*)&kOperandOff.v[M <= 2 ? M - 1 : 2][(4 * tid) & 127];
+    [[maybe_unused]] uint2 offw = make_uint2(0, 0);
+    if constexpr (NB == 1) {
+        if (out_dtype == 2) offw = *(const uint2*)&kOperandOff.v[M <= 2 ? M - 1 : 2][(4 * tid) & 127];
     }
     // Few rows are bound by latency: every load of the blocks and of the row's sum of squares is
     // issued before the first is used, from addresses that are always valid instead of under
@@ -363,12 +363,16 @@ __global__ __launch_bounds__(256) void k_norm_fwht(const float* __restrict__ src
 #pragma unroll
     for (int b = 0; b < NB; b++) {
         const int base = (blk0 + b) * 1024 + 4 * tid;
-        if (out_dtype == 2) {
-            if (M <= 2)
-                store_operand(v[b], offw, tid, blk0 + b, m, M, W, (uint8_t*)xs, (uint8_t*)out);
-            else
-                store_operand_wide(v[b], offw, tid, blk0 + b, m, M, W, (uint8_t*)xs, (uint8_t*)out);
-        } else if (out_dtype == 0) {
+        if constexpr (NB == 1) {                 // staged in xs: one block per workgroup
+            if (out_dtype == 2) {
+                if (M <= 2)
+                    store_operand(v[b], offw, tid, blk0, m, M, W, (uint8_t*)xs, (uint8_t*)out);
+                else
+                    store_operand_wide(v[b], offw, tid, blk0, m, M, W, (uint8_t*)xs, (uint8_t*)out);
+                return;
+            }
+        }
+        if (out_dtype == 0) {
             *(float4*)((float*)out + ro + base) = make_float4(v[b][0], v[b][1], v[b][2], v[b][3]);
         } else if (out_layout == 0) {
             typedef _Float16 h4 __attribute__((ext_vector_type(4)));
