@@ -82,6 +82,7 @@ __device__ inline uint32_t trits4(uint32_t w, uint32_t p3lo, uint32_t p3hi) {
 }
 
 using namespace gemm;
+using rg::barrier_lds;
 constexpr int kWStage = BN * 32;                     // staged packed bytes of one block of the tile rows
 constexpr int kSxOff = kTileBytes + 2 * kWStage;     // [kABuf][BM] fp32 row scales (with the A buffers)
 constexpr int kSwOff = kSxOff + kABuf * BM * 4;      // [2][BN] fp32 column scales (with the B buffers)
@@ -110,8 +111,8 @@ __device__ inline void fold_tile(v16f& acc, const v16i& I, float w, float sxv, s
 // the MFMAs of tile j + 1.  A wave's VALU does not overlap its own MFMAs; with two consumers
 // on each SIMD one's fold can run under the other's MFMAs (2.5 % faster than four consumers
 // of 64 rows; 64 x 64 per wave, fewer LDS reads, gains nothing over it).
-// Barriers as in the fp16 consumer: two before the first stage, one per stage (after the
-// stage's last LDS read).
+// Barriers: two before the first stage (the producers' first copies landed, stage 0 produced), one
+// per stage (after the stage's last LDS read).
 constexpr int kCW = 8;                   // consumer waves; each owns BM / kCW rows
 constexpr int kRH = BM / kCW;             // rows per consumer wave
 constexpr int kRT = kRH / 32;             // 32-row MFMA tiles per consumer wave
@@ -645,19 +646,17 @@ hipError_t launch_gemm_i8(const int8_t* A8, const float* SX, int ldS, const uint
         (void)hipGetLastError();
         p = plan(M, K, N, n_cu, false);
     }
-    if (p.k < kTall) {
-        rg::Mats P{};
-        P.W[0] = W;
-        P.C[0] = C;
-        P.N[0] = N;
-        P.ldc[0] = ldc;
-        for (int i = 1; i <= rg::kMaxMats; i++) P.g0[i] = 0x7fffffff;
-        const bool v4 = N % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)C & 15) == 0;
-        switch (p.k) {
-            case 0: return short_i8::launch_cfg<short_i8::Cfg<1>>(A8, SX, ldS, P, ws, c_dtype, v4, M, K, p.J, s);
-            case 1: return short_i8::launch_cfg<short_i8::Cfg<2>>(A8, SX, ldS, P, ws, c_dtype, v4, M, K, p.J, s);
-            default: return short_i8::launch_cfg<short_i8::Cfg<4>>(A8, SX, ldS, P, ws, c_dtype, v4, M, K, p.J, s);
-        }
+    rg::Mats P{};
+    P.W[0] = W;
+    P.C[0] = C;
+    P.N[0] = N;
+    P.ldc[0] = ldc;
+    for (int i = 1; i <= rg::kMaxMats; i++) P.g0[i] = 0x7fffffff;
+    const bool v4 = N % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)C & 15) == 0;
+    switch (p.k) {
+        case 0: return short_i8::launch_cfg<short_i8::Cfg<1>>(A8, SX, ldS, P, ws, c_dtype, v4, M, K, p.J, s);
+        case 1: return short_i8::launch_cfg<short_i8::Cfg<2>>(A8, SX, ldS, P, ws, c_dtype, v4, M, K, p.J, s);
+        case 2: return short_i8::launch_cfg<short_i8::Cfg<4>>(A8, SX, ldS, P, ws, c_dtype, v4, M, K, p.J, s);
     }
     if (c_dtype == 1)
         hipLaunchKernelGGL(k_gemm_ptq1_i8<true>, dim3(p.J.n_jobs), dim3(64 * (kCW + 4)), kLdsBytes, s, A8, SX, ldS, W, C, ldc, ws,
@@ -667,7 +666,7 @@ hipError_t launch_gemm_i8(const int8_t* A8, const float* SX, int ldS, const uint
                            ws, M, K, N, p.J);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return launch_pieces_sum<BM, BN>(ws, C, c_dtype, ldc, M, N, p.J, s);
+    return rg::launch_pieces_sum<BM, BN>(ws, P, c_dtype, v4, M, p.J, s);
 }
 
 }  // namespace kata

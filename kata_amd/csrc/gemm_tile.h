@@ -1,4 +1,4 @@
-// LDS tiles, copies and barriers of the tall int8 prefill GEMM (gemm_i8.hip): a workgroup of
+// LDS tiles and copies of the tall int8 prefill GEMM (gemm_i8.hip): a workgroup of
 // producer and consumer waves computes a 256 x 128 tile of C in stages of 128 bytes of k per
 // row.  The producers copy A tiles into LDS by DMA two stages ahead (three A buffers) and write
 // the decoded weights of the next stage into one of two B buffers; a stage is released by a
@@ -28,11 +28,6 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 __device__ inline uint32_t swz(int row, int chunk) { return (uint32_t)(row * ROWB + ((chunk ^ ((row >> 1) & 7)) << 4)); }
 __device__ inline uint8_t* tile_a(uint8_t* smem, int buf) { return smem + buf * (BM * ROWB); }
 __device__ inline uint8_t* tile_b(uint8_t* smem, int buf) { return smem + kABuf * BM * ROWB + buf * (BN * ROWB); }
-
-__device__ inline void barrier_lds() {
-    __builtin_amdgcn_s_waitcnt((15 & 15) | ((63 >> 4) << 14) | (7 << 4) | (0 << 8));   // lgkmcnt(0)
-    __builtin_amdgcn_s_barrier();
-}
 
 // Producer A copies: DMA instruction i of producer pw copies LDS bytes [1024 (4i + pw), +1024)
 // of stage st's A tile: lane l -> tile row r = 8 (4i + pw) + l / 8, LDS slot l % 8, which
