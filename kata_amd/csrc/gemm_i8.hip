@@ -589,9 +589,13 @@ hipError_t launch_cfg(const int8_t* A8, const float* SX, int ldS, const rg::Mats
 }  // namespace short_i8
 
 // The kernel of a call (k: of short_i8::kShapes, or kTall) and its schedule, with K pieces or
-// (pieces false) whole tiles only: the short tiles where the cost model has them cheaper than
-// the tall kernel's schedule (whole rounds of 256 x 128 tiles at 1.3 us per group, the rest in K
-// pieces); their row offsets are 32-bit.
+// (pieces false) whole tiles only: the short tiles, whose row offsets are 32-bit, where the cost model has
+// them cheaper than the tall kernel's whole rounds of 256 x 128 tiles at 3 + 1.3 us per group and the
+// rest in K pieces.  The tall model against measured us: 5120 -> 17408 55 / 56 - 57 up to 256 rows, 83 / 82 -
+// 85 at 512 (16 pieces); 17408 -> 5120 82 / 80 - 81 at 512, 180 / 174 at 1000.  It has K pieces of few
+// rows too long (17408 -> 5120 53 / 45 - 47 up to 256 rows): the choice is the faster kernel, or
+// within 2 % of it, at 35 of 36 sizes (41..1000 rows of four shapes); 200 rows of 5120 -> 5120 take 33
+// where the tall kernel takes 29.
 constexpr int kTall = 3;
 rg::Plan plan(int M, int K, int N, int n_cu, bool pieces) {
     const int nbk = K / kGroup;
