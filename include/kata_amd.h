@@ -138,7 +138,7 @@ int kata_gemv_q8_0_batch(int count, const uint8_t* const* W, float* const* y, co
                          int x_dtype, int K, int T, void* stream);
 
 /* ---------------------------------------------------------------- prefill ------------
- * Exact fp16 prefill GEMM with the ternary decode fused into the LDS tile load:
+ * Exact fp16 prefill GEMM, the ternary weights decoded into the matrix cores' operand registers:
  * C[m][n] = sum_k A[m][k] * half(trit[n][k] * d[n][k/128]), fp32 accumulation.
  * A is fp16 [M][lda] (lda >= K), C is [M][ldc] of c_dtype (KATA_F32 or KATA_F16).
  * K % 128 == 0; any M >= 1, N >= 1.

@@ -11,16 +11,17 @@
 //
 // What bounds it (K = 5120, N = 17408; before: 256 x 128 tiles whose producer waves wrote decoded
 // weights into LDS):
-//  * Many rows: power.  At 7300 rows every CU runs 256 x 256 tiles and the clock falls to 1.7 - 1.9
-//    of 2.4 GHz, so instructions and LDS bytes per MFMA count, not their latency: one wave per
-//    SIMD with 256 x 64 of C (2.7 vector instructions and half an LDS fragment read per MFMA)
-//    1337 -> 1100 us (1.18 PFLOP/s); a plain fp16 library product of the shape takes 1150.
-//    Two waves per SIMD of 128 x 64: 1118; of 128 x 32: 1220.
+//  * Many rows: at 7300 every CU runs 256 x 256 tiles, the clock falls to 1.7 - 2.0 of 2.4 GHz, and of
+//    a busy CU's cycles 62 - 65 % are MFMAs and 23 % other vector instructions, which with one wave per
+//    SIMD hardly overlap: instructions and LDS bytes per MFMA count, not their latency.  One wave per
+//    SIMD with 256 x 64 of C (2.8 vector instructions and half an LDS fragment read per MFMA) 1337 ->
+//    1100 us (1.18 PFLOP/s); a plain fp16 library product of the shape takes 1150.  Two waves per
+//    SIMD of 128 x 64: 1118; of 128 x 32: 1220.
 //  * A hundred to a few hundred rows: vector instructions and MFMAs of the two waves of a SIMD
 //    overlap only in part (the stage barrier keeps them in step): 128 x 256 tiles, 200 rows
 //    80 -> 61 us.
-//  * Up to 64 rows: the decode (about 2.5 vector instructions per weight, each weight once per
-//    launch) and the fixed 3 us to the first MFMA; short tiles instead of rows of padding: 41
+//  * Up to 64 rows: the decode (3 vector instructions per weight, each weight once per launch),
+//    waits (a third of the waves' time) and the fixed 3 us to the first MFMA; short tiles instead of rows of padding: 41
 //    rows 78 -> 28 us, 28 rows 78 -> 24 us.
 // Measured and not kept: trits from a conflict-free LDS table (half the vector instructions,
 // as many LDS cycles more: equal at 41 rows, 1.2x slower at 7300); waves of a SIMD in opposite

@@ -1,12 +1,12 @@
-// Exact fp16 prefill GEMM over a Q8_0 matrix with the decode fused into the LDS tile load:
-// the MTP head's K/V catch-up (Engine::encMtpKv, src/engine.cpp:392-401: k_expand_q8 then
+// Exact fp16 prefill GEMM over a Q8_0 matrix, the quants decoded into the MFMA's registers: the
+// MTP head's K/V catch-up (Engine::encMtpKv, src/engine.cpp:392-401: k_expand_q8 then
 // dGemm, shaders/mtp.metal:24-33).
 //
 // Semantics: C[m][n] = sum_k A[m][k] * half(d[n][k/32] * q[n][k]),  fp16 x fp16 -> fp32,
 // with half() round-to-nearest-even as the reference's expansion.  Every product term equals
 // the reference's; only the fp32 summation order differs (tolerance-based parity).
 //
-// Design: the skeleton of gemm_reg.h (tiles of 32, 64, 128 or 256 rows by 256 columns, weights
+// Design: the skeleton of gemm_reg.h (tiles of 64, 128 or 256 rows by 256 columns, weights
 // decoded straight into MFMA registers) with a Q8_0 decode:
 //  * Copies: a 128-k block is four 34-byte blocks of each of the tile's 256 weight rows (136 bytes,
 //    dword-aligned), copied into LDS by DMA one or two blocks ahead as nine 16-byte pieces (at
@@ -17,8 +17,9 @@
 //    rounds d * q once, to nearest even, as half(d * float(q)) does (the fp32 product of an
 //    fp16 and a 7-bit integer is exact).
 // What bounds it: up to a few hundred rows the packed bytes' way into LDS (36 KB a block, 5 DMA
-// instructions per wave, spread over the stages: 74.7 -> 66.7 us at 333 rows) and the 3 us to the
-// first MFMA; many rows the matrix cores at the clock that power leaves.  10240 -> 5120 / 5120 ->
+// instructions per wave, spread over the stages: 74.7 -> 66.7 us at 333 rows), bank conflicts (half the
+// LDS cycles: rows are 144 bytes apart) and the 3 us to the first MFMA; many rows the matrix cores and
+// the vector instructions beside them.  10240 -> 5120 / 5120 ->
 // 1024 before (256 x 128 tiles, decoded weights through LDS) -> now, us: 28 rows 45.9 / 16.4 ->
 // 23.1 / 11.9, 333 rows 77.5 / 23.1 -> 60.9 / 19.3, 512 rows 78.8 / 22.9 -> 77.5 / 21.7, 4000 rows
 // 491 / 64 -> 428 / 61.

@@ -1,6 +1,7 @@
 // Prefill GEMM skeleton with the weights decoded straight into MFMA operand registers
-// (gemm_f16.hip: PTQ1_0, gemm_q8.hip: Q8_0, gemm_i8.hip: int8, up to 128 rows).  C[M][N] = A[M][K] * W[N][K]^T, fp16 x fp16 -> fp32
-// (gemm_i8.hip has its own loop over the copies, waits and layouts here).
+// (gemm_f16.hip: PTQ1_0, gemm_q8.hip: Q8_0): C[M][N] = A[M][K] * W[N][K]^T, fp16 x fp16 -> fp32.  The
+// int8 GEMM's tiles of up to 128 rows (gemm_i8.hip) have their own loop over the copies, waits and
+// layouts here, and all of them share the cost model and the sum of K pieces.
 //
 // A workgroup of NWR x NWC waves computes a BM x BN tile of C; wave (wr, wc) owns 32 MT rows
 // and 32 NT columns as MT x NT tiles of v_mfma_f32_32x32x16_f16.  Lane l of the B operand
