@@ -164,13 +164,15 @@ typedef rg::Cfg<8, 2, 1, 4, 64, 2, 1, 1> Cfg256;     // 256 x 256
 typedef rg::Cfg<4, 1, 1, 8, 64, 2, 1, 2> Cfg128;     // 128 x 256
 typedef rg::Cfg<2, 1, 1, 8, 128, 2, 2, 2> Cfg64;     // 64 x 256
 typedef rg::Cfg<1, 1, 1, 8, 128, 2, 2, 2> Cfg32;     // 32 x 256
-// us per 128-k block of a tile, fitted to 25..7300 rows of the five model shapes; the schedule
-// that they choose is within 5 % of the best of all (tile, split) pairs at most of them.  Pieces of
-// fewer than 8 blocks from 15 % by the model: over 25..200 rows of twelve shapes (K 640..17408) what
-// they give falls short of what it has by up to 13 % (with / without, us: 25 rows of 1920 -> 1500
-// 9.5 / 17.7, of 5120 -> 1024 10.0 / 13.7; 64 rows of 4096 -> 4096 17.2 / 17.0, by the model 15.4 / 17.4).
+// us per 128-k block of a tile, fitted to 25..7300 rows of the five model shapes.  Pieces of fewer
+// than 8 blocks from 10 % by the model: of a gain that it has, up to 13 % of the time does not come
+// (64 rows of 4096 -> 4096 17.2 us with them, 17.0 without, by the model 15.4 / 17.4), and below
+// that the sums stay in longer pieces.  Over 1086 sizes (K 1024..17408, N 300..34816, 9..3000 rows)
+// what is chosen takes 1.8 % longer than the best schedule on average (1.5 % from any gain, 2.1 % from
+// 15 %), at one in a hundred 17 % or more.  With / without, us: 25 rows of 1920 -> 1500 9.5 / 17.7, of
+// 5120 -> 1024 10.0 / 13.7, 36 rows of 4736 -> 1882 11.0 / 15.4.
 constexpr int kBN = 256;
-constexpr float kShort = 0.85f;
+constexpr float kShort = 0.9f;
 constexpr rg::Shape kShapes[4] = {{32, kBN, 1.04f, 1.04f, kShort}, {64, kBN, 1.15f, 1.15f, kShort}, {128, kBN, 1.42f, 2.05f, kShort}, {256, kBN, 2.85f, 3.5f, kShort}};
 
 }  // namespace
