@@ -563,8 +563,8 @@ __global__ __launch_bounds__(512, 2) void k_gemm_i8_short(const int8_t* __restri
         }
 }
 
-// us per 128-group of a tile (see rg::Shape), fitted to 28..2500 rows of three model shapes
-constexpr rg::Shape kShapes[3] = {{32, 256, 1.1f, 1.1f, 1.0f}, {64, 256, 1.3f, 1.3f, 1.0f}, {128, 256, 1.75f, 1.8f, 1.0f}};
+// us per 128-group of a tile (see rg::Shape and plan below)
+constexpr rg::Shape kShapes[3] = {{32, 256, 1.02f, 1.02f, 1.0f}, {64, 256, 1.3f, 1.3f, 1.0f}, {128, 256, 1.9f, 1.9f, 1.0f}};
 
 template <class C>
 hipError_t launch_cfg(const int8_t* A8, const float* SX, int ldS, const rg::Mats& P, float* ws, int c_dtype, bool v4, int M,
@@ -590,12 +590,13 @@ hipError_t launch_cfg(const int8_t* A8, const float* SX, int ldS, const rg::Mats
 
 // The kernel of a call (k: of short_i8::kShapes, or kTall) and its schedule, with K pieces or
 // (pieces false) whole tiles only: the short tiles, whose row offsets are 32-bit, where the cost model has
-// them cheaper than the tall kernel's whole rounds of 256 x 128 tiles at 3 + 1.3 us per group and the
-// rest in K pieces.  The tall model against measured us: 5120 -> 17408 55 / 56 - 57 up to 256 rows, 83 / 82 -
-// 85 at 512 (16 pieces); 17408 -> 5120 82 / 80 - 81 at 512, 180 / 174 at 1000.  It has K pieces of few
-// rows too long (17408 -> 5120 53 / 45 - 47 up to 256 rows): the choice is the faster kernel, or
-// within 2 % of it, at 35 of 36 sizes (41..1000 rows of four shapes); 200 rows of 5120 -> 5120 take 33
-// where the tall kernel takes 29.
+// them cheaper than the tall kernel.  That: whole rounds of 256 x 128 tiles at 4 + 1.33 us per group,
+// then K pieces, whose sum costs 7 us and their bytes (whole tiles out, real rows back) at 6.2 TB/s.
+// Fitted together with kShapes to every schedule of 1086 sizes (K 1024..17408, N 300..34816, 9..3000
+// rows): what is chosen takes on average 0.4 %, and at one size in a hundred 9 % or more, longer than
+// the best, and is slower than the tall kernel by more than 3 % at 7 sizes, 9 % at most.  (Fitted
+// to a few shapes, with pieces at 4 us and 4 TB/s: 0.7 %, 13 %; 15 sizes, 18 %: 200 rows of 10240 ->
+// 2500 30.2 us against 25.2, of 5120 -> 5120 31.9 / 27.4; 1000 of 1024 -> 17408 61.9 / 52.7.)
 constexpr int kTall = 3;
 rg::Plan plan(int M, int K, int N, int n_cu, bool pieces) {
     const int nbk = K / kGroup;
@@ -605,8 +606,9 @@ rg::Plan plan(int M, int K, int N, int n_cu, bool pieces) {
         J = {J.G, T, 1, T};
     }
     const int rem = J.n_jobs - J.n_full;
-    double us = (J.n_full + n_cu - 1) / n_cu * (3.0 + nbk * 1.3);
-    if (rem) us += 3.0 + (nbk + J.S - 1) / J.S * 1.3 + 4.0 + (double)rem * BM * BN * 8.0 / 4e6;
+    const double rows = (double)M / ((M + BM - 1) / BM);                    // real rows per tile
+    double us = (J.n_full + n_cu - 1) / n_cu * (4.0 + nbk * 1.33);
+    if (rem) us += 4.0 + (nbk + J.S - 1) / J.S * 1.33 + 7.0 + rem * BN * (BM + rows) * 4.0 / 6.2e6;
     if (K <= (1 << 23)) {
         const rg::Plan t = rg::choose(short_i8::kShapes, M, (N + 255) / 256, nbk, n_cu, pieces);
         if (t.us < us) return t;

@@ -53,10 +53,10 @@ def _check_device(dev, M, K, N, bar):
 
 
 @pytest.mark.parametrize("rows,kind,M,K,N", [
-    (32, "split", 1, 1152, 700), (64, "whole", 1000, 384, 2050), (64, "split", 600, 3968, 257),
-    (64, "split", 41, 5120, 10240), (128, "whole", 257, 384, 17001), (128, "split", 600, 3968, 2050),
+    (32, "split", 1, 1152, 700), (64, "whole", 1000, 384, 2050), (64, "split", 1000, 1920, 700),
+    (64, "split", 41, 5120, 10240), (128, "whole", 257, 384, 17001), (128, "split", 257, 3968, 5120),
     (128, "split", 100, 5120, 12288), (128, "both", 700, 1152, 12001), (256, "whole", 513, 384, 8003),
-    (256, "split", 600, 5120, 2050), (256, "both", 400, 1152, 17001)])
+    (256, "split", 600, 5120, 2050), (256, "both", 1000, 1152, 9000)])
 def test_tile_heights(dev, rows, kind, M, K, N):
     """Every tile height with whole tiles, all tiles split and (128, 256) a split rest, ragged rows
     and columns, even and odd numbers of groups."""
@@ -74,8 +74,8 @@ def test_rows_beyond_32_bit_offsets(dev):
     _check_device(dev, 2, K - 128, 3, 7e-6)
 
 
-@pytest.mark.parametrize("rows,M,K,N", [(32, 1, 1408, 257), (64, 700, 2432, 700), (128, 65, 3200, 9000), (32, 20, 1408, 300),
-                                        (256, 50, 1408, 300), (256, 100, 1408, 300)])
+@pytest.mark.parametrize("rows,M,K,N", [(32, 1, 1408, 257), (32, 20, 1408, 300), (64, 1000, 1920, 700), (128, 257, 3968, 5120),
+                                        (256, 600, 3200, 2050)])
 def test_integer_sums_exact(dev, rows, M, K, N):
     """Unit scales: the exact integer sum, whatever the tile height and the split."""
     _plan_is(dev, M, K, N, rows, "split")
