@@ -246,7 +246,10 @@ __device__ inline void store_operand_wide(const float (&v)[4], uint2 offw, int t
 // one after the other: the row comes once from HBM and then from that XCD's L2.  x + y, norm to fp16, us with
 // the rows or the blocks of one row consecutive / so: 333 rows of 6144 18 / 19 / 8.9, 7300 rows
 // 468 / 362 / 188, 7300 rows of 17408 3555 / 1254 / 880; SwiGLU, 7300 rows of 17408, 250 / 224 / 220.
-template <int NB, bool NORM, bool ROW, bool ADD>
+// NR: 1024-blocks of the row whose loads are in flight together (for a shorter row its first block
+// again: free at widths 3072 and 4096, at 2048 four of six: 512 rows of x + y 5.2 us, 4.4 with NR 2,
+// 4.7 with the loads one by one).
+template <int NB, bool NORM, bool ROW, bool ADD, int NR = 1>
 __global__ __launch_bounds__(256) void k_norm_fwht(const float* __restrict__ src, const float* __restrict__ src2,
                                                    const float* __restrict__ gs, void* __restrict__ out, int out_dtype,
                                                    int out_layout, float* __restrict__ xnew,
@@ -280,7 +283,6 @@ __global__ __launch_bounds__(256) void k_norm_fwht(const float* __restrict__ src
     [[maybe_unused]] float s[NORM ? NB : 1][4];
     float inv = 1.0f;
     if constexpr (NORM) {
-        constexpr int NR = 6;                    // 1024-blocks of the row in flight
         const float* const yrow = ADD ? src2 + ro : nullptr;
         const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
         float4 ra[ROW ? 1 : NR], rc[ROW ? 1 : NR];
@@ -407,7 +409,8 @@ hipError_t launch_norm_fwht(const float* src, const float* src2, const float* gs
         constexpr bool ADD = decltype(add)::value;
         if (W == 1024) return go(k_norm_fwht<1, true, true, ADD>, dim3(M));
         if (W == 5120 && M > 200) return go(k_norm_fwht<5, true, true, ADD>, dim3(M));
-        return go(k_norm_fwht<1, true, false, ADD>, blocks);
+        if (W == 2048) return go(k_norm_fwht<1, true, false, ADD, 2>, blocks);
+        return go(k_norm_fwht<1, true, false, ADD, 6>, blocks);
     };
     return flags & 1 ? norm(std::true_type{}) : norm(std::false_type{});
 }

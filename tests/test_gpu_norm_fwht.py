@@ -87,7 +87,7 @@ def test_transform_feeds_the_gemv(dev):
     assert rel_l2(y, ref).max() < 2e-3
 
 
-@pytest.mark.parametrize("W,M", [(1024, 3), (1024, 9), (4096, 17), (5120, 8), (5120, 200), (5120, 201), (6144, 1), (7168, 5), (18432, 2)])
+@pytest.mark.parametrize("W,M", [(1024, 3), (1024, 9), (2048, 9), (4096, 17), (5120, 8), (5120, 200), (5120, 201), (6144, 1), (7168, 5), (18432, 2)])
 @pytest.mark.parametrize("add", [False, True])
 def test_norm_row_splits(dev, W, M, add):
     """Rows shorter and longer than the 6 blocks whose loads are in flight together, and both sides of
