@@ -164,16 +164,19 @@ typedef rg::Cfg<8, 2, 1, 4, 64, 2, 1, 1> Cfg256;     // 256 x 256
 typedef rg::Cfg<4, 1, 1, 8, 64, 2, 1, 2> Cfg128;     // 128 x 256
 typedef rg::Cfg<2, 1, 1, 8, 128, 2, 2, 2> Cfg64;     // 64 x 256
 typedef rg::Cfg<1, 1, 1, 8, 128, 2, 2, 2> Cfg32;     // 32 x 256
-// us per 128-k block of a tile, fitted to 25..7300 rows of the five model shapes.  Pieces of fewer
-// than 8 blocks from 10 % by the model: of a gain that it has, up to 13 % of the time does not come
-// (64 rows of 4096 -> 4096 17.2 us with them, 17.0 without, by the model 15.4 / 17.4), and below
-// that the sums stay in longer pieces.  Over 1086 sizes (K 1024..17408, N 300..34816, 9..3000 rows)
-// what is chosen takes 1.8 % longer than the best schedule on average (1.5 % from any gain, 2.1 % from
-// 15 %), at one in a hundred 17 % or more.  With / without, us: 25 rows of 1920 -> 1500 9.5 / 17.7, of
-// 5120 -> 1024 10.0 / 13.7, 36 rows of 4736 -> 1882 11.0 / 15.4.
+// us of a round and a 128-k block (rg::Shape), fitted to 1405 sizes (K 1024..17408, N 300..34816, 9..3000
+// rows): what they choose takes 0.9 % longer than the best schedule on average, and 13 % or more at one
+// size in a hundred.  Before, fitted to the model's shapes with tiles of 128 and 256 rows at 1.42 - 2.05
+// and 2.85 - 3.5 us by the busy CUs: 2.0 % and 19 % (1000 rows of 4096 -> 17408 173 us in 2.1 rounds of
+// 128-row tiles, against 149 in two and a split rest).
+// Pieces of fewer than 8 blocks only from 10 % by the model (from any gain: 0.7 % and 8 %): of a gain that
+// it has, up to 13 % of the time does not come (64 rows of 4096 -> 4096 17.2 us with them, 17.0 without,
+// by the model 15.4 / 17.4), and below that the sums stay in longer pieces.  With / without, us: 25
+// rows of 1920 -> 1500 9.5 / 17.7, of 5120 -> 1024 10.0 / 13.7.
 constexpr int kBN = 256;
 constexpr float kShort = 0.9f;
-constexpr rg::Shape kShapes[4] = {{32, kBN, 1.04f, 1.04f, kShort}, {64, kBN, 1.15f, 1.15f, kShort}, {128, kBN, 1.42f, 2.05f, kShort}, {256, kBN, 2.85f, 3.5f, kShort}};
+constexpr rg::Shape kShapes[4] = {{32, kBN, 3.0f, 1.04f, 1.04f, kShort}, {64, kBN, 3.0f, 1.15f, 1.15f, kShort},
+                                  {128, kBN, 3.0f, 1.48f, 1.48f, kShort}, {256, kBN, 7.0f, 2.6f, 2.6f, kShort}};
 
 }  // namespace
 

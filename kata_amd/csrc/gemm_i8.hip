@@ -563,8 +563,8 @@ __global__ __launch_bounds__(512, 2) void k_gemm_i8_short(const int8_t* __restri
         }
 }
 
-// us per 128-group of a tile (see rg::Shape and plan below)
-constexpr rg::Shape kShapes[3] = {{32, 256, 1.02f, 1.02f, 1.0f}, {64, 256, 1.3f, 1.3f, 1.0f}, {128, 256, 1.9f, 1.9f, 1.0f}};
+// us of a round and a 128-group (see rg::Shape and plan below)
+constexpr rg::Shape kShapes[3] = {{32, 256, 3.0f, 1.02f, 1.02f, 1.0f}, {64, 256, 3.0f, 1.3f, 1.3f, 1.0f}, {128, 256, 3.0f, 1.9f, 1.9f, 1.0f}};
 
 template <class C>
 hipError_t launch_cfg(const int8_t* A8, const float* SX, int ldS, const rg::Mats& P, float* ws, int c_dtype, bool v4, int M,

@@ -119,9 +119,11 @@ struct Q8F16 {
 typedef rg::Cfg<2, 1, 1, 8, 64, 2, 2, 2> Cfg64;      // 64 x 256
 typedef rg::Cfg<4, 1, 1, 8, 32, 3, 2, 2> Cfg128;     // 128 x 256
 typedef rg::Cfg<8, 2, 1, 4, 32, 3, 1, 1> Cfg256;     // 256 x 256
-// us per 128-k block of a tile, fitted to 28..2000 rows of 10240 -> 5120, 5120 -> 1024 and 17408
-// (a 32 row tile takes longer than a 64 row one here: its stages leave LDS for one ahead)
-constexpr rg::Shape kShapes[3] = {{64, 256, 1.5f, 1.55f, 1.0f}, {128, 256, 1.85f, 1.95f, 1.0f}, {256, 256, 3.3f, 3.5f, 1.0f}};
+// us of a round and a 128-k block (rg::Shape), fitted to 28..2000 rows of 10240 -> 5120, 5120 -> 1024
+// and 17408: over 1086 sizes (K 1024..17408, N 300..34816, 9..3000 rows) what they choose takes 0.6 %
+// longer than the best schedule on average, at one size in a hundred 9 % or more (a 32 row tile takes
+// longer than a 64 row one here: its stages leave LDS for one ahead)
+constexpr rg::Shape kShapes[3] = {{64, 256, 3.0f, 1.5f, 1.55f, 1.0f}, {128, 256, 3.0f, 1.85f, 1.95f, 1.0f}, {256, 256, 3.0f, 3.3f, 3.5f, 1.0f}};
 
 }  // namespace
 

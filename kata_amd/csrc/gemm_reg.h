@@ -349,12 +349,12 @@ inline hipError_t launch_pieces_sum(const float* ws, const Mats& P, int c_dtype,
 }
 
 // Schedules.  A configuration runs one workgroup per CU (8 waves, or 4 with the whole register
-// file) and is described by the microseconds a 128-k block of a tile takes on a mostly idle
-// chip (t_alone) and with every CU busy (t_full: the clock falls under full matrix load; in
-// between, in proportion to the busy CUs).
+// file) and is described by the microseconds in which a round of its tiles starts and stores and
+// those that a 128-k block of a tile takes on a mostly idle chip (t_alone) and with every CU busy
+// (t_full; in between, in proportion to the busy CUs).
 struct Shape {
     int bm, bn;
-    float t_alone, t_full;
+    float start, t_alone, t_full;
     float short_gain;    // all of a table alike, see choose
 };
 struct Plan {
@@ -365,7 +365,7 @@ struct Plan {
 constexpr int kPieceFloats = 2 * 256 * 128;               // workspace floats per CU
 // The cheapest schedule of T = row tiles x column groups tiles on n_cu workgroups: whole tiles
 // for the full rounds and the rest split S ways, or every tile split; a split costs the
-// pieces' way through memory and back (4 TB/s) and a launch (4 us); a round starts in 3 us.
+// pieces' way through memory and back (4 TB/s) and a launch (4 us).
 // Where every tile is split, pieces have at least min_blocks blocks.
 inline Plan plan(const Shape& c, int M, int G, int nbk, int n_cu, bool pieces, int min_blocks) {
     const long T = (long)((M + c.bm - 1) / c.bm) * G;
@@ -373,7 +373,7 @@ inline Plan plan(const Shape& c, int M, int G, int nbk, int n_cu, bool pieces, i
     auto part = [&](long jobs, int blocks) {                                // a set of equal jobs
         const long rounds = (jobs + n_cu - 1) / n_cu;
         const double busy = (double)jobs / (double)(rounds * n_cu);
-        return rounds * (3.0 + blocks * std::max((double)c.t_alone, c.t_full * busy));
+        return rounds * (c.start + blocks * std::max((double)c.t_alone, c.t_full * busy));
     };
     Plan best{{G, (int)T, 1, (int)T}, (float)part(T, nbk), 0};
     if (!pieces) return best;

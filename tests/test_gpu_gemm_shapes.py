@@ -70,10 +70,10 @@ def _device_weights(dev, K, N, seed, late):
 @pytest.mark.parametrize("late", [False, True])
 @pytest.mark.parametrize("rows,kind,M,K,N", [
     (32, "split", 1, 1152, 257), (64, "whole", 1000, 384, 2050), (64, "split", 513, 3968, 257),
-    (64, "both", 700, 3968, 12001), (128, "whole", 513, 384, 8003), (128, "split", 600, 3968, 2050),
-    (128, "both", 1000, 5120, 9000), (256, "whole", 400, 384, 17001), (256, "both", 1000, 5120, 17001)])
+    (128, "whole", 513, 384, 8003), (128, "split", 1000, 3968, 2050), (128, "both", 400, 1920, 17001),
+    (128, "both", 1000, 5120, 9000), (256, "whole", 700, 384, 12001), (256, "both", 1000, 5120, 17001)])
 def test_tile_heights(dev, rows, kind, M, K, N, late):
-    """Every tile height with whole tiles, all tiles split and a split rest, rows and columns ragged,
+    """Every tile height with whole tiles, all tiles split or (128, 256) a split rest, ragged rows and columns,
     even and odd numbers of blocks; every column by itself, so small ones count beside large, in
     units of the norm that a column of such products has (a lone sum may come out near zero)."""
     _plan_is(dev, "f16", M, K, N, rows, kind)

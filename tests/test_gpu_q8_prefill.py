@@ -120,7 +120,7 @@ def test_gemm_f16_tile_schedules(dev):
     called back to back so the workspace is reused with a different piece count; every
     output vs torch fp32 on the bit-exact expanded weights."""
     cases = [(256, 128, 128 * 256, "whole"),
-             (700, 3968, 12001, "both"),   # two rounds + 5 tiles of 16 pieces, ragged M and N
+             (700, 3968, 12001, "both"),   # a round + 26 tiles of 4 pieces, ragged M and N
              (41, 6144, 5120, "split"),    # 40 tiles of 6 pieces
              (1, 1152, 257, "split"),      # 2 tiles of 3 pieces
              (70, 1280, 200, "split")]
