@@ -3,7 +3,7 @@
 
     python bench.py [--steps K] [--warmup W] [--gpus 1] [--no-cpu] [--no-gemm]
 
-Workload (BASELINE.json configs[1], the batch-1 decode sweep): one step is the T=1 decode
+Workload (the batch-1 decode sweep): one step is the T=1 decode
 GEMV of every ternary matrix of one layer of each kind at the 27B shapes —
 GDN qkv 5120->10240, z 5120->6144, ssm_out 6144->5120; GQA q 5120->12288, k/v 5120->1024,
 o 6144->5120; FFN gate/up 5120->17408, down 17408->5120.  The matrices that multiply the
@@ -30,13 +30,13 @@ Also reported (same JSON line):
                duration, vs 8 TB/s HBM;
   per_matrix   GB/s of each matrix kind alone (200 repeats over rotating copies, replayed
                from one HIP graph so that the host's launch cost is not what is timed);
-  verify_t2    config 3: the T=2 verify GEMV on the FFN and attention shapes;
+  verify_t2    the T=2 verify GEMV on the FFN and attention shapes;
   verify_wide  the wide verification GEMV (T = 4, 8 token rows) on the same shapes;
-  q8_0_t1      config 3: the Q8_0 MTP-head GEMV, 17408x5120 and 5120x17408;
+  q8_0_t1      the Q8_0 MTP-head GEMV, 17408x5120 and 5120x17408;
   prefill_gemm pp512 exact fp16 GEMM TFLOPS (M=512, 5120->17408 and 17408->5120),
                vs 2.5 PFLOP/s dense fp16, the int8 variant, and the Q8_0 MTP K/V catch-up
                GEMM (eh_proj 10240->5120, wk 5120->1024, M=512);
-  cpu_baseline the reference's host path for BASELINE config 1 (the full 17408x5120 matrix:
+  cpu_baseline the reference's host path (the full 17408x5120 matrix:
                stage-loop dequantize_row_ptq1_0 + fp32 dot,
                oracle/kata_oracle.c:orc_cpu_gemv_ptq1_stage) on all host cores this process
                may use (nproc and the thread count stated), and on one thread.
@@ -99,7 +99,7 @@ LM_HEAD = (5120, (248320,))
 
 
 def run_config5(torch, ops, dev, stream):
-    """one bs=1 decode pass over all 64 layers + lm_head (5.6 GB of
+    """One bs=1 decode pass over all 64 layers + lm_head (5.6 GB of
     ternary weights, far above the Infinity Cache) and the 7300-token prefill GEMMs (as one
     GEMM and as 1024-row chunks), fp16 exact and int8 paths."""
     gen = torch.Generator(device=dev)
@@ -197,7 +197,7 @@ def run_config5(torch, ops, dev, stream):
 
 
 def cpu_baseline(threads: int, reps: int = 3):
-    """BASELINE config 1 on the host: the full 17408x5120 gate matrix, each row expanded by the
+    """On the host: the full 17408x5120 gate matrix, each row expanded by the
     reference's stage-loop dequantize_row_ptq1_0 then fp32 dots (orc_cpu_gemv_ptq1_stage),
     OpenMP over rows; best of `reps` runs, GB/s of packed bytes."""
     from oracle import oracle as orc
@@ -246,7 +246,7 @@ def sustain(torch, fn, stream, ms=200.0):
 
 
 def run_gemm(torch, ops, dev, stream, copies, ncopies):
-    """pp512 exact fp16 prefill GEMM (config 4): us and TFLOPS per shape, 30 calls over
+    """pp512 exact fp16 prefill GEMM: us and TFLOPS per shape, 30 calls over
     rotating weight copies between two events, after 200 ms of sustained calls."""
     gemm = {}
     M = 512
@@ -266,7 +266,7 @@ def run_gemm(torch, ops, dev, stream, copies, ncopies):
         tflops = 2.0 * M * N * K / (us * 1e-6) / 1e12
         gemm[name] = {"M": M, "K": K, "N": N, "us": round(us, 1), "TFLOPS": round(tflops, 1),
                       "frac": round(tflops / FP16_PEAK_TFLOPS, 4)}
-        # the int8 FFN variant (config 5): activation quantisation + int8 GEMM
+        # the int8 FFN variant: activation quantisation + int8 GEMM
         Q, SX = ops.quant_rows(A[K])
         sustain(torch, lambda: ops.gemm_ptq1_i8(Q, SX, copies[0][j], K, N, out=C), stream)
         a.record(stream)
@@ -772,7 +772,7 @@ def main():
     bytes_per_launch = set_bytes / launches
     achieved = bytes_per_launch / (gemv_launch_us * 1e-6) / 1e9
 
-    # ---- per matrix kind (config 2: 200 repeats each over rotating copies)
+    # ---- per matrix kind (200 repeats each over rotating copies)
     per_matrix = {}
     def time_reps(fn, nrep):
         return graph_time(torch, fn, nrep, stream, cap_stream)
@@ -793,7 +793,7 @@ def main():
     calib["ffn_gate_weight_stream_us"] = round(us_ws, 3)
     calib["ffn_gate_vs_weight_stream"] = round(per_matrix["ffn_gate"]["us"] / us_ws, 3)
 
-    # ---- config 3: T=2 speculative-verify GEMV (two fp16 activation columns
+    # ---- T=2 speculative-verify GEMV (two fp16 activation columns
     # shared per input) and the Q8_0 MTP-head GEMV (17408x5120 and 5120x17408, T=1)
     verify_t2 = {}
     for j, (name, K, N, grp) in enumerate(SWEEP):
@@ -836,10 +836,10 @@ def main():
     # ---- layer level: the FFN sublayer (27B shapes) through the dispatcher
     ffn = None if args.no_ffn else run_ffn(torch, ops, dev, stream, time_reps)
 
-    # ---- pp512 prefill GEMM (config 4), fp16 exact path
+    # ---- pp512 prefill GEMM, fp16 exact path
     gemm = None if args.no_gemm else run_gemm(torch, ops, dev, stream, copies, ncopies)
 
-    # ---- config 5: full 64-layer decode pass, M=7300 prefill
+    # ---- full 64-layer decode pass, M=7300 prefill
     cfg5 = None
     if not args.no_config5:
         cfg5 = run_config5(torch, ops, dev, stream)

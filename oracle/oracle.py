@@ -4,7 +4,7 @@ TEST INFRASTRUCTURE ONLY: imported by tests/, __graft_entry__.smoke() and bench.
 cpu_baseline leg, always as the checker or the timed CPU baseline.  The product path
 (kata_amd/) never imports this module.
 
-Also holds the seeded synthetic-data generators for the BASELINE configurations
+Also holds the seeded synthetic-data generators for the benchmark workloads
 (trits iid uniform on {-1,0,+1}, fp16 scales |N(0,0.02)|, fp16 N(0,1) activations,
 Q8_0 int8 uniform in [-127,127]).
 """

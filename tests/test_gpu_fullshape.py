@@ -69,7 +69,7 @@ def _q8_decode(W: torch.Tensor, K: int, N: int) -> torch.Tensor:
 
 @pytest.mark.parametrize("K,N", [(5120, 17408), (17408, 5120)])
 def test_q8_full_shape(dev, K, N):
-    """BASELINE config 3 Q8_0 MTP-head shapes, T = 1 and 2."""
+    """The Q8_0 MTP-head shapes, T = 1 and 2."""
     W_np, _, _ = orc.synth_q8(N, K, 400 + K)
     W = torch.from_numpy(W_np).to(dev)
     x_np = orc.synth_x(2, K, 401 + K)
@@ -86,7 +86,7 @@ def test_q8_full_shape(dev, K, N):
 
 
 def test_prefill_m7300_down_shape(dev):
-    """BASELINE config 5 prefill, the down projection (17408 -> 5120) at M = 7300, on the fp16
+    """Prefill, the down projection (17408 -> 5120) at M = 7300, on the fp16
     exact path and on the int8 path (the gate shape is in test_gpu_q8_prefill.py)."""
     M, K, N = 7300, 17408, 5120
     W_np, _, _ = orc.synth_ptq1(N, K, 5105)

@@ -99,7 +99,7 @@ def test_special_inputs(dev):
 
 
 def test_full_shape_17408x5120(dev):
-    """BASELINE config 1 shape: parity on sampled rows vs the oracle, and every row vs a
+    """The FFN gate shape: parity on sampled rows vs the oracle, and every row vs a
     torch fp32 product of the GPU-expanded (bit-exact) weights."""
     K, N = 5120, 17408
     W_np, _, _ = orc.synth_ptq1(N, K, 2026)

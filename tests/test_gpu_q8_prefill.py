@@ -97,7 +97,7 @@ def test_gemm_f16_random(dev, M, K, N):
 
 @pytest.mark.parametrize("K,N", [(5120, 17408), (17408, 5120)])
 def test_gemm_f16_pp512_full_shape(dev, K, N):
-    """BASELINE config 4 shapes: every row vs torch fp32 on the bit-exact expanded weights,
+    """The FFN shapes at 512 rows: every row vs torch fp32 on the bit-exact expanded weights,
     plus oracle rows; fp16 output within fp16 rounding of the fp32 output."""
     M = 512
     W_np, _, _ = orc.synth_ptq1(N, K, K ^ N)
@@ -141,7 +141,7 @@ def test_gemm_f16_tile_schedules(dev):
 
 @pytest.mark.parametrize("M", [1024, 7300])
 def test_gemm_config5_prefill_shapes(dev, M):
-    """BASELINE config 5 prefill: a 7300-token prompt as one GEMM and as the reference's
+    """Prefill: a 7300-token prompt as one GEMM and as the reference's
     1024-row chunk, gate shape, on the fp16 exact path and on the int8 FFN path.  References:
     torch fp32 on the bit-exact expanded weights; for int8 the per-group integer sums come
     from fp32 matmuls of integer values (exact below 2^24) and fold in ascending group order."""
